@@ -658,86 +658,205 @@ __global__ void __launch_bounds__(kBlock)
 // Chopped spatial binning of the references of candidate tasks.  A
 // reference counts one entry (c0) in its first bin and one exit (c1) in its
 // last, and grows the box of every bin it spans with the triangle clipped to
-// that bin, so a bin can hold a box without counts.  Blocks spanning at most
-// kLdsTasks tasks bin in LDS and merge every touched bin.
+// that bin, so a bin can hold a box without counts.
 __device__ __forceinline__ bool sp_evaluated(const SDec* dec, const uint32_t* cand_excl,
                                              int32_t t) {
     return dec[t].cand && cand_excl[t] < kMaxCand;
 }
 
+// References per block of a level of at most `tasks` tasks and `refs`
+// references: near the root long runs divide the blocks that merge into each
+// bin, while at least 256 (512 past the first levels) of them remain; deeper,
+// about one task's references, so that a run spans few windows of tasks.
+// 1M references, levels 0 / 8 / 12 / 17: 143 / 95 / 159 / 888 us at 2048
+// references a block, 205 / 85 / 95 / 296 at 512, 458 / 151 / 107 / 132 at
+// 128, 854 / 203 / 166 / 128 at 64.
+inline uint32_t sp_run(uint32_t tasks, uint32_t refs) {
+    const uint32_t cap = tasks <= 16 ? std::min(2048u, refs / 256) : std::min(512u, refs / 512);
+    return std::max(64u, std::min(cap, refs / tasks));
+}
+
+// The instructions themselves: fminf / fmaxf put a canonicalising v_max in
+// front of every operand that comes from memory or a select.
+__device__ __forceinline__ float vmin(float a, float b) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float vmax(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float vmin3(float a, float b, float c) {
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float vmax3(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+// Where a triangle's edges cross one plane of axis u: whether any does, and
+// the bounds of the crossings on the other two axes (empty without one).
+struct Crossing {
+    bool any;
+    float vmn, vmx, wmn, wmx;
+};
+
+__device__ __forceinline__ Crossing no_crossing() {
+    return Crossing{false, 3.0e38f, -3.0e38f, 3.0e38f, -3.0e38f};
+}
+
+__device__ __forceinline__ Crossing cross_plane(const float (&pu)[3], const float (&pv)[3],
+                                                const float (&pw)[3], float plane) {
+    Crossing c = no_crossing();
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int j = (i + 1) % 3;
+        if (!((pu[i] < plane && pu[j] > plane) || (pu[i] > plane && pu[j] < plane))) continue;
+        const float t = (plane - pu[i]) / (pu[j] - pu[i]);
+        const float qv = pv[i] + t * (pv[j] - pv[i]);
+        const float qw = pw[i] + t * (pw[j] - pw[i]);
+        c.any = true;
+        c.vmn = vmin(c.vmn, qv);
+        c.vmx = vmax(c.vmx, qv);
+        c.wmn = vmin(c.wmn, qw);
+        c.wmx = vmax(c.wmx, qw);
+    }
+    return c;
+}
+
+__device__ __forceinline__ void grow_axis(Acc* g, int k, float mn, float mx) {
+    if (!(mn <= mx)) return;
+    atomicMin(&g->mn[k], fenc(mn));
+    atomicMax(&g->mx[k], fenc(mx));
+}
+
+// A thread takes one (reference, axis) pair and walks the bins the reference
+// spans along that axis; neighbouring bins share a plane, so each plane's
+// crossings are found once (the values are clip_box's, operation by
+// operation).  The block's run of references is binned in LDS, kLdsTasks
+// tasks at a time (a level's references are ordered by task): a task that
+// lies inside the run is then stored, another merged by atomics.
+// Near the root the time is the atomics on the few tasks' bins, at the deep
+// levels the windows' latency (clear, bin, flush).  A thread per reference
+// that added to global bins where a run spans more than kLdsTasks tasks made
+// up to 300 device atomics per reference: 4.2 ms of a 100,003-triangle build
+// (514 us at its widest level), 1.0 ms (68 us) this way, the same bins.
+// Measured and not used: a wave per run with one lane per (axis, bin) and no
+// atomics, 1.4 ms (every lane clips every reference).
 __global__ void __launch_bounds__(kBlock)
-    sp_bin_kernel(const SLevel* L, const SRef* refs, const SDec* dec, const uint32_t* cand_excl,
-                  const float* verts, uint32_t prim_count, Acc* sbins, uint32_t run) {
+    sp_bin_kernel(const SLevel* L, const SRef* refs, const STask* tasks, const SDec* dec,
+                  const uint32_t* cand_excl, const float* verts, uint32_t prim_count, Acc* sbins,
+                  uint32_t run) {
     __shared__ Acc s_b[kLdsTasks][3 * kBins];
-    __shared__ int32_t s_t0, s_nt;
-    const uint32_t nrefs = L->nrefs;
+    __shared__ uint32_t s_slot[kLdsTasks];  // bins of each task of the window, or kNoSlot
+    const uint32_t nrefs = L->nrefs, num_tasks = L->num_tasks;
     const uint32_t first = blockIdx.x * run;
     if (first >= nrefs || L->cand_total == 0) return;  // whole block
     const uint32_t end = first + run < nrefs ? first + run : nrefs;
-    if (threadIdx.x == 0) {
-        int32_t nt = 0;
-        s_t0 = block_tasks(refs, first, end, &nt);
-        s_nt = nt;
-    }
-    for (uint32_t k = threadIdx.x; k < uint32_t(kLdsTasks * 3 * kBins); k += kBlock)
-        acc_clear(s_b[k / (3 * kBins)][k % (3 * kBins)]);
-    __syncthreads();
-    const int32_t t0 = s_t0;
-    for (uint32_t i = first + threadIdx.x; i < end; i += kBlock) {
-        const SRef r = refs[i];
-        const int32_t t = r.task;
-        if (t >= 0 && sp_evaluated(dec, cand_excl, t) && r.prim < prim_count) {
-            const SDec& d = dec[t];
-            Acc* base = in_run(t, t0, s_nt) ? s_b[t - t0]
-                                            : sbins + size_t(cand_excl[t]) * 3 * kBins;
-            const float* v = verts + size_t(r.prim) * 9;
-            for (int ax = 0; ax < 3; ++ax) {
-                const float org = sel3(d.org, ax), inv = sel3(d.inv, ax);
-                const uint32_t b0 = bin_of(sel3(r.mn, ax), org, inv);
-                const uint32_t b1 = max(b0, bin_of(sel3(r.mx, ax), org, inv));
-                atomicAdd(&base[ax * kBins + b0].c0, 1u);
-                atomicAdd(&base[ax * kBins + b1].c1, 1u);
-                for (uint32_t b = b0; b <= b1 && b < uint32_t(kBins); ++b) {
-                    float mn[3], mx[3];
-                    if (b0 == b1) {
-                        for (int k = 0; k < 3; ++k) {
-                            mn[k] = r.mn[k];
-                            mx[k] = r.mx[k];
-                        }
-                    } else {
-                        const float lo = b == b0 ? -3.0e38f : d.org[ax] + float(b) * d.width[ax];
-                        const float hi =
-                            b == b1 ? 3.0e38f : d.org[ax] + float(b + 1) * d.width[ax];
-                        if (!clip_box(v, ax, lo, hi, r.mn, r.mx, mn, mx)) continue;
-                    }
-                    Acc* g = &base[ax * kBins + b];
-                    for (int k = 0; k < 3; ++k) {
-                        if (!(mn[k] <= mx[k])) continue;
-                        atomicMin(&g->mn[k], fenc(mn[k]));
-                        atomicMax(&g->mx[k], fenc(mx[k]));
-                    }
-                }
-            }
-        }
-    }
-    __syncthreads();
-    if (t0 >= 0)
-        for (uint32_t k = threadIdx.x; k < uint32_t(s_nt * 3 * kBins); k += kBlock) {
-            const uint32_t tt = k / (3 * kBins), slot = k % (3 * kBins);
-            const int32_t t = t0 + int32_t(tt);
-            if (!sp_evaluated(dec, cand_excl, t)) continue;
-            const Acc& a = s_b[tt][slot];
-            const uint32_t empty = fenc(1e34f);
-            if ((a.c0 | a.c1) == 0 && a.mn[0] == empty && a.mn[1] == empty && a.mn[2] == empty)
+    const uint32_t task_first = uint32_t(refs[first].task), task_last = uint32_t(refs[end - 1].task);
+    for (uint32_t w = task_first; w <= task_last && w < num_tasks; w += kLdsTasks) {
+        const uint32_t wn = min(uint32_t(kLdsTasks), min(task_last, num_tasks - 1) - w + 1);
+        const uint32_t a = max(first, tasks[w].begin), b = min(end, tasks[w + wn - 1].end);
+        if (threadIdx.x < wn)
+            s_slot[threadIdx.x] = sp_evaluated(dec, cand_excl, int32_t(w + threadIdx.x))
+                                      ? cand_excl[w + threadIdx.x]
+                                      : kNoSlot;
+        for (uint32_t k = threadIdx.x; k < wn * 3 * kBins; k += kBlock)
+            acc_clear(s_b[k / (3 * kBins)][k % (3 * kBins)]);
+        __syncthreads();
+        const uint32_t count = b > a ? b - a : 0u;
+        for (uint32_t q = threadIdx.x; q < 3 * count; q += kBlock) {
+            const uint32_t ax = q < count ? 0u : (q < 2 * count ? 1u : 2u);
+            const SRef* r = refs + (a + q - ax * count);
+            const uint32_t t = uint32_t(r->task) - w, prim = r->prim;
+            if (t >= wn || s_slot[t] == kNoSlot || prim >= prim_count) continue;
+            const uint32_t ay = ax == 2 ? 0u : ax + 1, az = ax == 0 ? 2u : ax - 1;
+            const SDec& d = dec[w + t];
+            const float org = d.org[ax], inv = d.inv[ax], width = d.width[ax];
+            const float umn = r->mn[ax], umx = r->mx[ax];
+            const float vmn = r->mn[ay], vmx = r->mx[ay], wmn = r->mn[az], wmx = r->mx[az];
+            const uint32_t b0 = bin_of(umn, org, inv);
+            const uint32_t b1 = max(b0, bin_of(umx, org, inv));
+            Acc* g = &s_b[t][ax * kBins + b0];
+            atomicAdd(&g->c0, 1u);
+            atomicAdd(&g[b1 - b0].c1, 1u);
+            if (b0 == b1) {
+                grow_axis(g, int(ax), umn, umx);
+                grow_axis(g, int(ay), vmn, vmx);
+                grow_axis(g, int(az), wmn, wmx);
                 continue;
-            Acc* g = &sbins[size_t(cand_excl[t]) * 3 * kBins + slot];
-            if (a.c0) atomicAdd(&g->c0, a.c0);
-            if (a.c1) atomicAdd(&g->c1, a.c1);
-            for (int q = 0; q < 3; ++q) {
-                atomicMin(&g->mn[q], a.mn[q]);
-                atomicMax(&g->mx[q], a.mx[q]);
+            }
+            float pu[3], pv[3], pw[3];
+            const float* v = verts + size_t(prim) * 9;
+            for (int i = 0; i < 3; ++i) {
+                pu[i] = v[i * 3 + ax];
+                pv[i] = v[i * 3 + ay];
+                pw[i] = v[i * 3 + az];
+            }
+            // the crossings' rounding on the other axes, a few ulps of the
+            // vertices' magnitude (clip_box)
+            const float ev = vmax3(fabsf(pv[0]), fabsf(pv[1]), fabsf(pv[2])) * 0x1p-20f + 1e-30f;
+            const float ew = vmax3(fabsf(pw[0]), fabsf(pw[1]), fabsf(pw[2])) * 0x1p-20f + 1e-30f;
+            Crossing low = no_crossing();
+            for (uint32_t bin = b0; bin <= b1; ++bin, ++g) {
+                const bool top = bin == b1;
+                const float lo = bin == b0 ? -3.0e38f : org + float(bin) * width;
+                const float hi = top ? 3.0e38f : org + float(bin + 1) * width;
+                const Crossing high = top ? no_crossing() : cross_plane(pu, pv, pw, hi);
+                float omn[3] = {3.0e38f, vmin(low.vmn, high.vmn), vmin(low.wmn, high.wmn)};
+                float omx[3] = {-3.0e38f, vmax(low.vmx, high.vmx), vmax(low.wmx, high.wmx)};
+                if (low.any) {
+                    omn[0] = lo;
+                    omx[0] = lo;
+                }
+                if (high.any) {
+                    omn[0] = vmin(omn[0], hi);
+                    omx[0] = hi;
+                }
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+                    if (pu[i] >= lo && pu[i] <= hi) {
+                        omn[0] = vmin(omn[0], pu[i]);
+                        omx[0] = vmax(omx[0], pu[i]);
+                        omn[1] = vmin(omn[1], pv[i]);
+                        omx[1] = vmax(omx[1], pv[i]);
+                        omn[2] = vmin(omn[2], pw[i]);
+                        omx[2] = vmax(omx[2], pw[i]);
+                    }
+                low = high;
+                const float cu0 = vmax3(omn[0], lo, umn), cu1 = vmin3(omx[0], hi, umx);
+                const float cv0 = vmax(omn[1] - ev, vmn), cv1 = vmin(omx[1] + ev, vmx);
+                const float cw0 = vmax(omn[2] - ew, wmn), cw1 = vmin(omx[2] + ew, wmx);
+                if (!(cu0 <= cu1 && cv0 <= cv1 && cw0 <= cw1)) continue;
+                grow_axis(g, int(ax), cu0, cu1);
+                grow_axis(g, int(ay), cv0, cv1);
+                grow_axis(g, int(az), cw0, cw1);
             }
         }
+        __syncthreads();
+        for (uint32_t k = threadIdx.x; k < wn * 3 * kBins; k += kBlock) {
+            const uint32_t t = k / (3 * kBins), slot = k % (3 * kBins);
+            if (s_slot[t] == kNoSlot) continue;
+            const Acc& o = s_b[t][slot];
+            Acc* g = &sbins[size_t(s_slot[t]) * 3 * kBins + slot];
+            if (tasks[w + t].begin >= first && tasks[w + t].end <= end) {
+                *g = o;
+                continue;
+            }
+            if (o.c0) atomicAdd(&g->c0, o.c0);
+            if (o.c1) atomicAdd(&g->c1, o.c1);
+            for (int c = 0; c < 3; ++c) {
+                if (o.mn[c] != fenc(1e34f)) atomicMin(&g->mn[c], o.mn[c]);
+                if (o.mx[c] != fenc(-1e34f)) atomicMax(&g->mx[c], o.mx[c]);
+            }
+        }
+        __syncthreads();
+    }
 }
 
 // Best spatial split of each evaluated candidate (list: their tasks);
@@ -1253,6 +1372,8 @@ ResultCode gpu_build_spatial(const RTAabb* aabbs, const float* centers, size_t s
                                  : tb <= kRunMidTasks      ? kRunMid
                                                            : uint32_t(kBlock);
             const uint32_t bg = (ref_bound + run - 1) / run;
+            const uint32_t per = sp_run(tb, ref_bound);
+            const uint32_t spg = (ref_bound + per - 1) / per;
             const uint32_t tg = (tb + kBlock - 1) / kBlock;
             const uint32_t gg = std::min<uint32_t>((tb + kBlock / kBins - 1) / (kBlock / kBins),
                                                    kSplitGrid);  // task groups
@@ -1279,8 +1400,8 @@ ResultCode gpu_build_spatial(const RTAabb* aabbs, const float* centers, size_t s
                 return fail(e, "spatial candidate scan");
             hipLaunchKernelGGL(cand_clear_kernel, dim3(cg), dim3(kBlock), 0, stream, L, cand,
                                cand_list, dup, sbins);
-            hipLaunchKernelGGL(sp_bin_kernel, dim3(bg), dim3(kBlock), 0, stream, L, rc, dec, cand,
-                               verts, n, sbins, run);
+            hipLaunchKernelGGL(sp_bin_kernel, dim3(spg), dim3(kBlock), 0, stream, L, rc, tc, dec,
+                               cand, verts, n, sbins, per);
             hipLaunchKernelGGL(sp_split_kernel, dim3(sg), dim3(kBlock), 0, stream, L, cand_list,
                                tc, dec, sbins, dup);
             if ((e = scan_exclusive_dev(ScanArrays{{dup}}, 1, ScanCounts{{&L->num_tasks}}, tb,

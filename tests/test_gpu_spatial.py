@@ -215,3 +215,16 @@ def test_spatial_errors():
         b.construct_spatial_sah(_dev(verts[:5]))
     with pytest.raises(rt.BuildError):
         rt.Builder(_dev(centers[:0])).construct_spatial_sah(_dev(verts[:0]))
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 1023, 20_011])
+def test_spatial_binning_runs(n):
+    """Sizes around the binning's runs of 64 references and its windows of 16
+    tasks: long slivers span many bins, and tasks cross the ends of runs."""
+    verts = slivers(n, length=0.4, seed=n)
+    bvh = _build(verts, "spatial")
+    _check_structure(bvh, n)
+    if n >= 1023:  # a few dozen slivers may find no plane cheaper than an object split
+        assert bvh.index_count > n
+    rays8 = ray_set(verts, 2000, seed=n, kind="box")
+    _hits_all_paths(bvh, verts, rays8)
