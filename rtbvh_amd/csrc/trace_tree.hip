@@ -274,12 +274,11 @@ __device__ void make_node(const LevelArgs& a, uint32_t b, uint32_t w, QItem* qou
 // ---- compressed 8-wide nodes -------------------------------------------
 
 // A slot candidate: a binary interior node, a binary leaf of several
-// primitives (opened into them when they fit), or one primitive (an index
-// position, with the bounds of its triangle).
+// primitives (a node of its own), or one primitive (an index position, with
+// the bounds of its triangle).
 struct Cand {
     int32_t id;
-    int32_t kind;  // 0 interior, 1 leaf of n > 1 primitives, 2 primitive
-    uint32_t n;
+    bool prim;
     float lo[3], hi[3];
 };
 
@@ -291,8 +290,7 @@ __device__ __forceinline__ bool cand_prim(const LevelArgs& a, uint32_t pos, Cand
                                           const DevAabb& leaf) {
     if (pos >= a.index_count) return false;
     c.id = int32_t(pos);
-    c.kind = 2;
-    c.n = 1;
+    c.prim = true;
     const uint32_t prim = a.indices[pos];
     if (prim < a.prim_count) {
         const float* v = a.verts + size_t(prim) * 9;
@@ -318,84 +316,10 @@ __device__ __forceinline__ bool cand_prim(const LevelArgs& a, uint32_t pos, Cand
     return true;
 }
 
-// Appends binary node i as a candidate (an empty leaf adds nothing).
-__device__ bool cand_binary(const LevelArgs& a, int32_t i, Cand* c, int& ns) {
-    if (i < 0 || uint32_t(i) >= a.node_count) return false;
-    DevAabb n;
-    ldn(a.nodes + i, n);
-    if (n.extra1 == 0) return true;
-    if (ns >= kWide) return false;
-    if (n.extra1 == 1) return cand_prim(a, uint32_t(n.extra2), c[ns++], n);
-    Cand& d = c[ns++];
-    d.id = i;
-    d.kind = n.extra1 > 1 ? 1 : 0;
-    d.n = n.extra1 > 1 ? uint32_t(n.extra1) : 0u;
-    for (int k = 0; k < 3; ++k) {
-        d.lo[k] = n.min[k];
-        d.hi[k] = n.max[k];
-    }
-    return n.extra2 >= 0;
-}
-
-// The candidates of one compressed node held in registers: an append
-// shifts every entry down one place and writes the new one at the end, so
-// after ns appends they sit at [kWide - ns, kWide) in order, and every write
-// is by a compile-time index (an access by a run-time index would place
-// the arrays in scratch memory).
-struct CandRegs {
-    int32_t id[kWide], kind[kWide];
-    uint32_t n[kWide];
-    float lo0[kWide], lo1[kWide], lo2[kWide], hi0[kWide], hi1[kWide], hi2[kWide];
-
-    __device__ __forceinline__ void push(const Cand& t) {
-#pragma unroll
-        for (int q = 0; q + 1 < kWide; ++q) {
-            id[q] = id[q + 1];
-            kind[q] = kind[q + 1];
-            n[q] = n[q + 1];
-            lo0[q] = lo0[q + 1];
-            lo1[q] = lo1[q + 1];
-            lo2[q] = lo2[q + 1];
-            hi0[q] = hi0[q + 1];
-            hi1[q] = hi1[q + 1];
-            hi2[q] = hi2[q + 1];
-        }
-        id[kWide - 1] = t.id;
-        kind[kWide - 1] = t.kind;
-        n[kWide - 1] = t.n;
-        lo0[kWide - 1] = t.lo[0];
-        lo1[kWide - 1] = t.lo[1];
-        lo2[kWide - 1] = t.lo[2];
-        hi0[kWide - 1] = t.hi[0];
-        hi1[kWide - 1] = t.hi[1];
-        hi2[kWide - 1] = t.hi[2];
-    }
-};
-
-// Binary node i as one candidate t (add: whether it gives one; an empty
-// leaf gives none): cand_binary for a caller that stores the candidate.
-__device__ __forceinline__ bool cand_binary1(const LevelArgs& a, int32_t i, Cand& t, bool& add) {
-    add = false;
-    if (i < 0 || uint32_t(i) >= a.node_count) return false;
-    DevAabb n;
-    ldn(a.nodes + i, n);
-    if (n.extra1 == 0) return true;
-    add = true;
-    if (n.extra1 == 1) return cand_prim(a, uint32_t(n.extra2), t, n);
-    t.id = i;
-    t.kind = n.extra1 > 1 ? 1 : 0;
-    t.n = n.extra1 > 1 ? uint32_t(n.extra1) : 0u;
-    for (int k = 0; k < 3; ++k) {
-        t.lo[k] = n.min[k];
-        t.hi[k] = n.max[k];
-    }
-    return n.extra2 >= 0;
-}
-
 // Grid of one axis: origin p at least one step below lo, step 2^(e-127) a
 // power of two with (hi - lo) / step <= 252 and step >= 2^-22 * max(|lo|,
 // |hi|) (so the spare step outlasts float rounding in the traversal).
-__device__ bool grid_axis(float lo, float hi, float& p, uint32_t& ebyte, double& step) {
+__device__ bool grid_axis(float lo, float hi, float& p, uint32_t& ebyte) {
     const double ext = double(hi) - double(lo);
     const double mag = fmax(fabs(double(lo)), fabs(double(hi)));
     double need = fmax(ext / 252.0, mag * 0x1p-22);
@@ -405,8 +329,7 @@ __device__ bool grid_axis(float lo, float hi, float& p, uint32_t& ebyte, double&
     if (m == 0.5) --k;                 // need is itself a power of two
     if (k + 127 < 1 || k + 127 > 254) return false;
     ebyte = uint32_t(k + 127);
-    step = ldexp(1.0, k);
-    const double pd = double(lo) - step;
+    const double pd = double(lo) - ldexp(1.0, k);
     float pf = float(pd);
     if (double(pf) > pd) pf = nextafterf(pf, -3.4028235e38f);
     p = pf;
@@ -435,260 +358,303 @@ __device__ __forceinline__ uint32_t dp_decision(const uint32_t* dpd, uint32_t k,
     return (dpd[k] >> (4u * (j - 1u))) & 15u;
 }
 
+// Blocks of the node kernel: same-address atomics serialize (about 10 ns
+// each), so that one per wave of eight nodes made a level of 63,000 nodes
+// take 250 us; a block of 128 nodes claims its ranges at once.
+constexpr int kNodeBlock = 1024;
+constexpr int kNodeWaves = kNodeBlock / 64;
+struct NodeShared {
+    uint32_t inner[kNodeWaves], tris[kNodeWaves];
+    uint32_t base[3];
+};
+
+// The 8 lanes of a node's group: a value of one of them, their votes.
+template <typename T>
+__device__ __forceinline__ T group_get(T v, uint32_t lane) {
+    return __shfl(v, int(lane), kWide);
+}
+
+__device__ __forceinline__ uint32_t group_votes(bool v) {
+    return uint32_t(__ballot(v) >> (threadIdx.x & 56u)) & 0xFFu;
+}
+
 // One compressed node from queue item (b, w).  Its slots come from the
 // SAH-optimal distribution of b's subtree over eight slots (dp_level_kernel):
 // b's children get k and 8 - k slots, and each part either stays one slot
 // or spreads further.  The slots are then placed so that slot s lies towards
 // the octant s (bit k of s set: the + side of axis k) of the node's centre,
 // greedily by alignment; a ray whose direction has signs O visits keys
-// s ^ O in increasing order, the near side first.  Called by all 64 lanes
-// of a wave (`live` false: no item): the wide-node, triangle and queue
-// counters take one atomic per wave, the lanes' offsets from wave scans.
-__device__ void make_node8(const LevelArgs& a, bool live, uint32_t b, uint32_t w, QItem* qout,
-                           uint32_t* qout_count) {
-    CandRegs cr;
-    int ns = 0;
-    const auto append = [&](const Cand& t) {
-        cr.push(t);
-        ++ns;
-    };
-    bool ok = live;
-    if (ok && (b >= a.node_count || w >= a.wcap)) {
-        atomicOr(&a.counters[2], 1u);
-        ok = false;
-    }
-    DevAabb bn;
-    if (ok) ldn(a.nodes + b, bn);
-    if (!ok) {
-        // nothing to gather
-    } else if (bn.extra1 >= 0) {  // a root that is a leaf, or a leaf of several primitives
-        if (bn.extra1 > kWide || bn.extra2 < 0) ok = false;
-        for (int32_t j = 0; ok && j < bn.extra1; ++j)
-        {
-            Cand t;
-            ok = cand_prim(a, uint32_t(bn.extra2 + j), t, bn);
-            append(t);
-        }
-    } else {
-        // (binary node, slots) pairs still to place; at most 8 are pending
-        uint32_t st_node[kWide], st_slots[kWide];
-        int sp = 0;
-        const uint32_t k8 = dp_decision(a.dpd, b, 8u);
-        if (bn.extra2 < 0 || k8 == 0u || k8 >= 8u) {
-            ok = false;
+// s ^ O in increasing order, the near side first.
+//
+// Eight lanes build a node, one per slot (`live`, b and w are theirs; every
+// thread of the block calls): a part of j slots owns j consecutive lanes, so
+// the parts of a node spread at the same time, each lane gathers, quantizes
+// and stores its own slot, and the placement takes one reduction per slot.
+// A node's time is the chain of loads down its subtree, so a level of one
+// node takes 11 us and one of 20,000 about 20 us; the two widest levels of a
+// 1M tree (63,000 nodes) take 61 us each.  With one thread per node, which
+// walked the parts, placed and quantized the slots one after another, they
+// took 27, 60 and 100 us (level kernels of a 1M build 926 us, now 470; of a
+// batch of 48 scenes with 1M triangles 895, now 365).  Blocks of 512 threads
+// measured the same, at most 64 registers (8 waves per SIMD) spilled and
+// lost 10 %.
+__device__ void make_node8(const LevelArgs& a, NodeShared& sh, bool live, uint32_t b, uint32_t w,
+                           QItem* qout, uint32_t* qout_count) {
+    const uint32_t lane = threadIdx.x & 7u;
+    bool bad = live && (b >= a.node_count || w >= a.wcap);
+    const bool run = live && !bad;
+    DevAabb nd;  // of the part in hand; its box bounds the part's triangles
+    for (int k = 0; k < 3; ++k) nd.min[k] = nd.max[k] = 0.0f;
+    nd.extra1 = nd.extra2 = 0;
+    if (run) ldn(a.nodes + b, nd);
+    // the part that starts at this lane: slots 0, none
+    uint32_t node = 0, slots = 0, prims = 0;
+    bool open = false;  // its decision is still to be taken
+    if (run) {
+        if (nd.extra1 >= 0) {  // a root that is a leaf, or a leaf of several primitives
+            if (nd.extra1 > kWide || nd.extra2 < 0)
+                bad = true;
+            else if (lane == 0) {
+                slots = kWide;
+                prims = uint32_t(nd.extra1);
+            }
         } else {
-            st_node[sp] = uint32_t(bn.extra2) + 1u;
-            st_slots[sp++] = 8u - k8;
-            st_node[sp] = uint32_t(bn.extra2);
-            st_slots[sp++] = k8;
-        }
-        while (ok && sp > 0) {
-            --sp;
-            const uint32_t n = st_node[sp], j = st_slots[sp];
-            if (n >= a.node_count || j < 1u || j > 8u) {
-                ok = false;
-                break;
-            }
-            DevAabb nd;
-            ldn(a.nodes + n, nd);
-            const uint32_t d = dp_decision(a.dpd, n, j);
-            if (nd.extra1 >= 0 && d == kDissolve) {  // its primitives, one slot each
-                if (nd.extra2 < 0 || uint32_t(nd.extra1) > j) {
-                    ok = false;
-                    break;
-                }
-                for (int32_t q = 0; ok && q < nd.extra1; ++q) {
-                    Cand t;
-                    ok = ns < kWide && cand_prim(a, uint32_t(nd.extra2 + q), t, nd);
-                    if (ok) append(t);
-                }
-            } else if (nd.extra1 >= 0 || d == 0u) {  // one slot
-                Cand t;
-                bool add = false;
-                ok = cand_binary1(a, int32_t(n), t, add);
-                if (ok && add) {
-                    if (ns >= kWide)
-                        ok = false;
-                    else
-                        append(t);
-                }
-            } else {  // spread over j slots: k to the left child, j - k to the right
-                if (nd.extra2 < 0 || d >= j || sp + 2 > kWide) {
-                    ok = false;
-                    break;
-                }
-                st_node[sp] = uint32_t(nd.extra2) + 1u;
-                st_slots[sp++] = j - d;
-                st_node[sp] = uint32_t(nd.extra2);
-                st_slots[sp++] = d;
+            const uint32_t k8 = dp_decision(a.dpd, b, 8u);
+            if (nd.extra2 < 0 || k8 == 0u || k8 >= 8u) {
+                bad = true;
+            } else if (lane == 0 || lane == k8) {
+                node = uint32_t(nd.extra2) + (lane ? 1u : 0u);
+                slots = lane ? 8u - k8 : k8;
+                open = true;
             }
         }
     }
-    if (live && (!ok || ns == 0)) atomicOr(&a.counters[2], 1u);
-    ok = ok && ns > 0;
-    // bounds of the node and the centre of every candidate
-    float lo[3] = {0.0f, 0.0f, 0.0f}, hi[3] = {0.0f, 0.0f, 0.0f};
-    if (ok) {
-        // the candidates sit at [kWide - ns, kWide); fminf / fmaxf skip NaN as
-        // a fold from the first candidate would
-        for (int k = 0; k < 3; ++k) {
-            lo[k] = __builtin_inff();
-            hi[k] = -__builtin_inff();
-        }
-#pragma unroll
-        for (int j = 0; j < kWide; ++j)
-            if (j >= kWide - ns) {
-                lo[0] = fminf(lo[0], cr.lo0[j]);
-                lo[1] = fminf(lo[1], cr.lo1[j]);
-                lo[2] = fminf(lo[2], cr.lo2[j]);
-                hi[0] = fmaxf(hi[0], cr.hi0[j]);
-                hi[1] = fmaxf(hi[1], cr.hi1[j]);
-                hi[2] = fmaxf(hi[2], cr.hi2[j]);
+    // every round takes the open parts' decisions; a part that spreads gives
+    // the lane after its left share to its right child
+    while (__ballot(open) != 0) {
+        uint32_t split = 0;
+        if (open) {
+            open = false;
+            if (node >= a.node_count || slots < 1u || slots > 8u) {
+                bad = true;
+                slots = 0;
+            } else {
+                ldn(a.nodes + node, nd);
+                const uint32_t d = dp_decision(a.dpd, node, slots);
+                if (nd.extra1 >= 0 && d == kDissolve) {  // its primitives, one slot each
+                    if (nd.extra2 < 0 || uint32_t(nd.extra1) > slots)
+                        bad = true;
+                    else
+                        prims = uint32_t(nd.extra1);
+                } else if (nd.extra1 < 0 && d != 0u) {  // d slots to the left child
+                    if (nd.extra2 < 0 || d >= slots)
+                        bad = true;
+                    else
+                        split = d;
+                }
             }
-        for (int k = 0; k < 3; ++k)
-            if (!(isfinite(lo[k]) && isfinite(hi[k]) && lo[k] <= hi[k])) ok = false;
-        if (!ok) atomicOr(&a.counters[2], 2u);
+        }
+        const uint32_t starts = group_votes(slots != 0);
+        const uint32_t mine = starts & ((2u << lane) - 1u);
+        const uint32_t owner = mine ? 31u - uint32_t(__builtin_clz(mine)) : lane;
+        const uint32_t o_split = group_get(split, owner), o_slots = group_get(slots, owner);
+        const uint32_t o_child = group_get(uint32_t(nd.extra2), owner);
+        if (o_split != 0 && lane == owner + o_split) {
+            node = o_child + 1u;
+            slots = o_slots - o_split;
+            open = true;
+        }
+        if (split != 0) {
+            node = uint32_t(nd.extra2);
+            slots = split;
+            open = true;
+        }
+    }
+    // this lane's candidate: a primitive of a dissolved leaf, or the part
+    // that starts here
+    Cand c;
+    c.id = 0;
+    c.prim = false;
+    for (int k = 0; k < 3; ++k) c.lo[k] = c.hi[k] = 0.0f;
+    bool has = false;
+    {
+        const uint32_t starts = group_votes(slots != 0);
+        const uint32_t mine = starts & ((2u << lane) - 1u);
+        const uint32_t owner = mine ? 31u - uint32_t(__builtin_clz(mine)) : lane;
+        const uint32_t o_prims = group_get(prims, owner);
+        const uint32_t o_first = group_get(uint32_t(nd.extra2), owner);
+        DevAabb leaf;
+        for (int k = 0; k < 3; ++k) {
+            leaf.min[k] = group_get(nd.min[k], owner);
+            leaf.max[k] = group_get(nd.max[k], owner);
+        }
+        if (run && o_prims != 0) {
+            if (lane - owner < o_prims) {
+                has = true;
+                if (!cand_prim(a, o_first + (lane - owner), c, leaf)) bad = true;
+            }
+        } else if (run && slots != 0 && nd.extra1 != 0) {  // an empty leaf gives nothing
+            has = true;
+            if (nd.extra1 == 1) {
+                if (!cand_prim(a, uint32_t(nd.extra2), c, nd)) bad = true;
+            } else {
+                c.id = int32_t(node);
+                if (nd.extra2 < 0) bad = true;
+                for (int k = 0; k < 3; ++k) {
+                    c.lo[k] = nd.min[k];
+                    c.hi[k] = nd.max[k];
+                }
+            }
+        }
+    }
+    const uint32_t cands = group_votes(has);
+    bool ok = run && group_votes(bad) == 0 && cands != 0;
+    if (live && !ok && lane == 0) atomicOr(&a.counters[2], 1u);
+    // bounds of the node: fminf / fmaxf skip NaN
+    float lo[3], hi[3];
+    for (int k = 0; k < 3; ++k) {
+        lo[k] = has ? c.lo[k] : __builtin_inff();
+        hi[k] = has ? c.hi[k] : -__builtin_inff();
+        for (int off = 1; off < kWide; off <<= 1) {
+            lo[k] = fminf(lo[k], __shfl_xor(lo[k], off, kWide));
+            hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], off, kWide));
+        }
+    }
+    // the grid: lane k takes axis k
+    float p[3];
+    uint32_t eb[3];
+    {
+        const uint32_t ax = lane < 2u ? lane : 2u;
+        const float l = ax == 0 ? lo[0] : (ax == 1 ? lo[1] : lo[2]);
+        const float h = ax == 0 ? hi[0] : (ax == 1 ? hi[1] : hi[2]);
+        float pa = 0.0f;
+        uint32_t ea = 0;
+        bool good = ok && isfinite(l) && isfinite(h) && l <= h;
+        if (good) good = grid_axis(l, h, pa, ea);
+        if (ok && group_votes(!good) != 0) {
+            if (lane == 0) atomicOr(&a.counters[2], 2u);
+            ok = false;
+        }
+        for (uint32_t k = 0; k < 3; ++k) {
+            p[k] = group_get(pa, k);
+            eb[k] = group_get(ea, k);
+        }
     }
     // octant placement: each round takes the first (candidate, free slot)
-    // pair of the highest alignment score.  Every loop over candidates and
-    // slots is unrolled, so nothing is indexed at run time.
-    float off0[kWide], off1[kWide], off2[kWide];
+    // pair of the highest alignment score
+    uint32_t slot = 0, taken = 0;
+    {
+        float sc[kWide];
+        float off[3];
+        for (int k = 0; k < 3; ++k) off[k] = (c.lo[k] + c.hi[k]) - (lo[k] + hi[k]);
 #pragma unroll
-    for (int k = 0; k < kWide; ++k) {
-        const bool v = ok && k >= kWide - ns;
-        off0[k] = v ? (cr.lo0[k] + cr.hi0[k]) - (lo[0] + hi[0]) : 0.0f;
-        off1[k] = v ? (cr.lo1[k] + cr.hi1[k]) - (lo[1] + hi[1]) : 0.0f;
-        off2[k] = v ? (cr.lo2[k] + cr.hi2[k]) - (lo[2] + hi[2]) : 0.0f;
-    }
-    uint32_t cand_slot[kWide];  // the slot of each candidate
+        for (int s = 0; s < kWide; ++s)
+            sc[s] = ((s & 1) ? off[0] : -off[0]) + ((s & 2) ? off[1] : -off[1]) +
+                    ((s & 4) ? off[2] : -off[2]);
+        bool waiting = ok && has;
+        while (__ballot(waiting) != 0) {
+            // lowest (candidate, slot) among equal scores; a NaN score loses
+            float best = -__builtin_inff();
+            uint32_t pair = waiting ? (lane << 3) | uint32_t(__builtin_ctz(~taken)) : 0x100u;
 #pragma unroll
-    for (int k = 0; k < kWide; ++k) cand_slot[k] = 0;
-    uint32_t placed = 0, taken = 0;  // candidates placed, slots taken
-    for (int it = 0; ok && it < ns; ++it) {
-        float best = -3.4e38f;
-        int bk = -1, bs = -1;
+            for (int s = kWide - 1; s >= 0; --s)
+                if (waiting && !(taken & (1u << s)) && sc[s] >= best) {
+                    best = sc[s];
+                    pair = (lane << 3) | uint32_t(s);
+                }
 #pragma unroll
-        for (int k = 0; k < kWide; ++k) {
-            if (k < kWide - ns || (placed & (1u << k))) continue;
-#pragma unroll
-            for (int s = 0; s < kWide; ++s) {
-                if (taken & (1u << s)) continue;
-                const float sc = ((s & 1) ? off0[k] : -off0[k]) +
-                                 ((s & 2) ? off1[k] : -off1[k]) +
-                                 ((s & 4) ? off2[k] : -off2[k]);
-                if (bk < 0 || sc > best) {
-                    best = sc;
-                    bk = k;
-                    bs = s;
+            for (int o = 1; o < kWide; o <<= 1) {
+                const float ob = __shfl_xor(best, o, kWide);
+                const uint32_t op = __shfl_xor(pair, o, kWide);
+                if (ob > best || (ob == best && op < pair)) {
+                    best = ob;
+                    pair = op;
                 }
             }
-        }
-#pragma unroll
-        for (int k = 0; k < kWide; ++k)
-            if (k == bk) cand_slot[k] = uint32_t(bs);
-        placed |= 1u << bk;
-        taken |= 1u << bs;
-    }
-    // grid, children and triangles
-    float p[3] = {0.0f, 0.0f, 0.0f};
-    uint32_t eb[3] = {0u, 0u, 0u};
-    double step[3] = {1.0, 1.0, 1.0};
-    for (int k = 0; ok && k < 3; ++k)
-        if (!grid_axis(lo[k], hi[k], p[k], eb[k], step[k])) {
-            atomicOr(&a.counters[2], 2u);
-            ok = false;
-        }
-    double inv_step[3];
-    for (int k = 0; k < 3; ++k) inv_step[k] = 1.0 / step[k];
-    uint32_t n_inner = 0, n_tris = 0;
-#pragma unroll
-    for (int j = 0; j < kWide; ++j) {
-        if (!(ok && j >= kWide - ns)) continue;
-        if (cr.kind[j] == 2)
-            ++n_tris;
-        else
-            ++n_inner;
-    }
-    // offsets: wave scans of the lanes' counts, one atomic per counter and
-    // wave (the last lane's inclusive sums are the wave's totals)
-    const uint32_t inc_i = wave_inclusive(n_inner), inc_t = wave_inclusive(n_tris);
-    uint32_t wb = 0, tb = 0, qb = 0;
-    if ((threadIdx.x & 63u) == 63u) {
-        wb = inc_i ? atomicAdd(&a.counters[0], inc_i) : 0u;
-        tb = inc_t ? atomicAdd(&a.counters[1], inc_t) : 0u;
-        qb = inc_i ? atomicAdd(qout_count, inc_i) : 0u;
-    }
-    wb = __shfl(wb, 63, 64);
-    tb = __shfl(tb, 63, 64);
-    qb = __shfl(qb, 63, 64);
-    if (!ok) return;
-    const uint32_t wbase = wb + inc_i - n_inner, tbase = tb + inc_t - n_tris;
-    const uint32_t qbase = qb + inc_i - n_inner;
-    if (wbase + n_inner > a.wcap || tbase + n_tris > a.index_count) {
-        atomicOr(&a.counters[2], 1u);
-        return;
-    }
-    DevCw8Node m;
-    m.px = p[0];
-    m.py = p[1];
-    m.pz = p[2];
-    // slot masks first: the triangles and the inner children are stored in
-    // slot order, each at its rank among the slots of its kind
-    uint32_t imask = 0, lmask = 0;
-#pragma unroll
-    for (int k = 0; k < kWide; ++k) {
-        if (k < kWide - ns) continue;
-        if (cr.kind[k] == 2)
-            lmask |= 1u << cand_slot[k];
-        else
-            imask |= 1u << cand_slot[k];
-    }
-    uint32_t qlo[3][2] = {{0u, 0u}, {0u, 0u}, {0u, 0u}};
-    uint32_t qhi[3][2] = {{0u, 0u}, {0u, 0u}, {0u, 0u}};
-#pragma unroll
-    for (int s = 0; s < kWide; ++s)  // empty slots: an inverted box, never entered
-        if (!((imask | lmask) & (1u << s)))
-            for (int ax = 0; ax < 3; ++ax) qlo[ax][s >> 2] |= 255u << ((s & 3) * 8);
-#pragma unroll
-    for (int k = 0; k < kWide; ++k) {
-        if (k < kWide - ns) continue;
-        const uint32_t sl = cand_slot[k], sh = (sl & 3u) * 8u, below = (1u << sl) - 1u;
-        const float clo[3] = {cr.lo0[k], cr.lo1[k], cr.lo2[k]};
-        const float chi[3] = {cr.hi0[k], cr.hi1[k], cr.hi2[k]};
-        for (int ax = 0; ax < 3; ++ax) {
-            const uint32_t ql = quant_lo(clo[ax], p[ax], inv_step[ax]) << sh;
-            const uint32_t qh = quant_hi(chi[ax], p[ax], inv_step[ax]) << sh;
-            if (sl >= 4u) {
-                qlo[ax][1] |= ql;
-                qhi[ax][1] |= qh;
-            } else {
-                qlo[ax][0] |= ql;
-                qhi[ax][0] |= qh;
+            if (waiting && (pair >> 3) == lane) {
+                slot = pair & 7u;
+                waiting = false;
             }
+            if (pair < 0x40u) taken |= 1u << (pair & 7u);
         }
-        if (cr.kind[k] == 2) {
-            write_tri(a.tris, tbase + uint32_t(__popc(lmask & below)), a.verts, a.prim_count,
-                      a.indices[cr.id[k]], a.scene_off, a.scenes);
-        } else {
-            const uint32_t r = uint32_t(__popc(imask & below));
-            qout[qbase + r].b = uint32_t(cr.id[k]);
-            qout[qbase + r].w = wbase + r;
+        // the lanes without a candidate take the slots left over, in order
+        uint32_t left = ~taken & 0xFFu;
+        uint32_t skip = uint32_t(__popc(~cands & ((1u << lane) - 1u)));
+        for (; skip > 0; --skip) left &= left - 1u;
+        if (!has) slot = left ? uint32_t(__builtin_ctz(left)) : 0u;
+    }
+    // offsets: the votes below this group within the wave, the waves before
+    // it within the block, one atomic per block for the wide nodes and
+    // triangles together (two words of one 64-bit sum) and one for the queue
+    const bool is_tri = ok && has && c.prim, is_inner = ok && has && !c.prim;
+    const uint64_t inner = __ballot(is_inner), tris = __ballot(is_tri);
+    const uint32_t wave = threadIdx.x >> 6;
+    if ((threadIdx.x & 63u) == 0u) {
+        sh.inner[wave] = uint32_t(__popcll(inner));
+        sh.tris[wave] = uint32_t(__popcll(tris));
+    }
+    __syncthreads();
+    uint32_t inner_before = 0, tris_before = 0, ni = 0, nt = 0;
+    for (uint32_t k = 0; k < uint32_t(kNodeWaves); ++k) {
+        if (k == wave) {
+            inner_before = ni;
+            tris_before = nt;
         }
+        ni += sh.inner[k];
+        nt += sh.tris[k];
     }
-    m.emask = eb[0] | (eb[1] << 8) | (eb[2] << 16) | (imask << 24);
-    m.child_base = wbase;
-    m.tri_base = tbase;
-    m.lmask = lmask;
-    m.pad = 0;
-    for (int word = 0; word < 2; ++word) {
-        m.qlo_x[word] = qlo[0][word];
-        m.qlo_y[word] = qlo[1][word];
-        m.qlo_z[word] = qlo[2][word];
-        m.qhi_x[word] = qhi[0][word];
-        m.qhi_y[word] = qhi[1][word];
-        m.qhi_z[word] = qhi[2][word];
+    if (threadIdx.x == 0) {
+        const unsigned long long both =
+            atomicAdd(reinterpret_cast<unsigned long long*>(a.counters),
+                      (unsigned long long)ni | ((unsigned long long)nt << 32));
+        sh.base[0] = uint32_t(both);
+        sh.base[1] = uint32_t(both >> 32);
+        sh.base[2] = ni ? atomicAdd(qout_count, ni) : 0u;
     }
-    a.cnodes[w] = m;
+    __syncthreads();
+    const uint64_t groups_below = (1ull << (threadIdx.x & 56u)) - 1ull;
+    const uint32_t below_i = inner_before + uint32_t(__popcll(inner & groups_below));
+    const uint32_t wbase = sh.base[0] + below_i, qbase = sh.base[2] + below_i;
+    const uint32_t tbase = sh.base[1] + tris_before + uint32_t(__popcll(tris & groups_below));
+    const uint32_t n_inner = uint32_t(__popc(group_votes(is_inner)));
+    const uint32_t n_tris = uint32_t(__popc(group_votes(is_tri)));
+    if (ok && (wbase + n_inner > a.wcap || tbase + n_tris > a.index_count)) {
+        if (lane == 0) atomicOr(&a.counters[2], 1u);
+        ok = false;
+    }
+    // slot masks: the triangles and the inner children are stored in slot
+    // order, each at its rank among the slots of its kind
+    uint32_t imask = is_inner ? 1u << slot : 0u, lmask = is_tri ? 1u << slot : 0u;
+    for (int o = 1; o < kWide; o <<= 1) {
+        imask |= __shfl_xor(imask, o, kWide);
+        lmask |= __shfl_xor(lmask, o, kWide);
+    }
+    if (!ok) return;
+    DevCw8Node* m = a.cnodes + w;
+    uint8_t* q = reinterpret_cast<uint8_t*>(m->qlo_x) + slot;
+#pragma unroll
+    for (int ax = 0; ax < 3; ++ax) {
+        // empty slots: an inverted box, never entered; 1 / step is exact
+        const double inv_step = ldexp(1.0, 127 - int(eb[ax]));
+        q[ax * 8] = has ? uint8_t(quant_lo(c.lo[ax], p[ax], inv_step)) : uint8_t(255);
+        q[24 + ax * 8] = has ? uint8_t(quant_hi(c.hi[ax], p[ax], inv_step)) : uint8_t(0);
+    }
+    const uint32_t below = (1u << slot) - 1u;
+    if (is_tri) {
+        write_tri(a.tris, tbase + uint32_t(__popc(lmask & below)), a.verts, a.prim_count,
+                  a.indices[c.id], a.scene_off, a.scenes);
+    } else if (is_inner) {
+        const uint32_t r = uint32_t(__popc(imask & below));
+        qout[qbase + r].b = uint32_t(c.id);
+        qout[qbase + r].w = wbase + r;
+    }
+    if (lane == 0) {
+        float4* h = reinterpret_cast<float4*>(m);
+        h[0] = make_float4(p[0], p[1], p[2],
+                           __uint_as_float(eb[0] | (eb[1] << 8) | (eb[2] << 16) | (imask << 24)));
+        h[1] = make_float4(__uint_as_float(wbase), __uint_as_float(tbase), __uint_as_float(lmask),
+                           0.0f);
+    }
 }
 
 // ---- SAH-optimal distribution of binary subtrees over compressed slots ---
@@ -843,21 +809,23 @@ __global__ void __launch_bounds__(kBlock)
 
 // clear: the queue count two levels ahead (the level before's input, read
 // by nobody now) is zeroed for the level after this one to count into.
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kNodeBlock)
     level8_kernel(LevelArgs a, const QItem* qin, const uint32_t* qin_count, QItem* qout,
                   uint32_t* qout_count, uint32_t* clear, uint32_t level) {
+    __shared__ NodeShared sh;
     const uint32_t q = *qin_count;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         *clear = 0;
         if (q > 0) atomicMax(&a.counters[4], level + 1);  // levels with work
     }
-    // whole blocks iterate together: make_node8 needs every lane of a wave
-    for (uint32_t base = blockIdx.x * kBlock; base < q; base += gridDim.x * kBlock) {
-        const uint32_t i = base + threadIdx.x;
+    // whole blocks iterate together: make_node8 needs every thread
+    constexpr uint32_t kNodes = kNodeBlock / kWide;
+    for (uint32_t base = blockIdx.x * kNodes; base < q; base += gridDim.x * kNodes) {
+        const uint32_t i = base + threadIdx.x / kWide;
         QItem it;
         it.b = it.w = 0;
         if (i < q) it = qin[i];
-        make_node8(a, i < q, it.b, it.w, qout, qout_count);
+        make_node8(a, sh, i < q, it.b, it.w, qout, qout_count);
     }
 }
 
@@ -985,6 +953,7 @@ hipError_t enqueue_setup(const TraceTreePlan* t, const DeviceBvh& tree, hipStrea
 }
 
 constexpr uint32_t kBinGrid = 2048;   // persistent blocks per distribution-level kernel
+constexpr uint32_t kNodeGrid = 512;      // persistent blocks per compressed-node level
 constexpr uint32_t kBinLevelGrid = 512;  // blocks of kBinBlock per breadth-first level
 
 void enqueue_bin_level(const TraceTreePlan* t, const DeviceBvh& tree, uint32_t level,
@@ -1010,7 +979,7 @@ void enqueue_level(const TraceTreePlan* t, const LevelArgs& a, uint32_t level, u
     const int in = level & 1, outq = in ^ 1;  // queue buffers alternate
     uint32_t* w = t->words;
     if (t->width == 8)
-        hipLaunchKernelGGL(level8_kernel, dim3(grid), dim3(kBlock), 0, stream, a, t->q[in],
+        hipLaunchKernelGGL(level8_kernel, dim3(kNodeGrid), dim3(kNodeBlock), 0, stream, a, t->q[in],
                            w + qword(level), t->q[outq], w + qword(level + 1),
                            w + qword(level + 2), level);
     else

@@ -202,3 +202,20 @@ def test_batch_errors():
     with pytest.raises(rt.RTBvhError, match="InvalidArgument"):
         rt._lib.check(rt._lib.lib().rtbvh_gpu_intersect_batch(
             batch._h, rays.data_ptr(), roff.data_ptr(), 64, out.data_ptr(), 1, None), "flags")
+
+
+@pytest.mark.parametrize("scene_count", [2, 127, 128, 129, 300])
+def test_batch_of_tiny_scenes_around_a_block_of_nodes(scene_count):
+    """The compressed tree's first level holds one node per scene and is built
+    128 nodes to a block, eight lanes to a node: scenes of 3 to 12 triangles
+    give nodes of 3 to 8 slots, with and without children."""
+    vl = [scenes.random_soup(3 + s % 10, 0.3, seed=500 + s) for s in range(scene_count)]
+    batch, verts, offs = _build_batch(vl)
+    batch.attach_triangles(_dev(verts))
+    rays_l = [ray_set(v, 24, seed=900 + s, kind="box") for s, v in enumerate(vl)]
+    roff = rt.SceneBatch.ray_offsets([len(r) for r in rays_l], "cuda")
+    got = batch.intersect(_dev(np.concatenate(rays_l)), roff).cpu().numpy()
+    got = got.view(ref.HIT).reshape(-1)
+    for s, v in enumerate(vl):
+        want = ref.trace_brute(v, as_rays(rays_l[s]))
+        assert hits_equal(got[24 * s:24 * s + 24], want).all(), s
