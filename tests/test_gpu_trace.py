@@ -285,3 +285,30 @@ def test_ray_packets_unpack_and_trace():
     want = ref.trace_mbvh(m, idx, verts, as_rays(rays8[: 4 * p]), mode=ref.MODE_LOWEST_ID,
                           threads=8)
     assert hits_equal(hp.view(ref.HIT).reshape(-1), want).all()
+
+
+@pytest.mark.parametrize("rays_n", [1, 65, 5000, 1_300_000])
+@pytest.mark.parametrize("per_leaf", [1, 24])
+def test_vertex_traversals_over_ray_counts_and_leaf_sizes(rays_n, per_leaf):
+    """The traversals over the caller's vertex array hand out rays one per
+    lane up to two per resident lane (about a million), in ranges per wave
+    beyond, and test a leaf's triangles one per iteration: every count of
+    rays, leaves of 1 to 24 triangles, both tie rules and any hit."""
+    verts = scenes.random_soup(700, 0.2, seed=17)
+    aabbs, centers = prep(verts)
+    bvh = rt.Builder(_dev(centers), aabbs=_dev(flat(aabbs)),
+                     primitives_per_leaf=per_leaf).construct_binned_sah()
+    mbvh = rt.Mbvh.from_bvh(bvh)
+    nodes = bvh.nodes().cpu().numpy().view(ref.AABB).reshape(-1)
+    quads = mbvh.quad_nodes().cpu().numpy().view(ref.MBVH).reshape(-1)
+    idx = bvh.indices().cpu().numpy().view(np.uint32)
+    rays8 = ray_set(verts, rays_n, seed=18 + rays_n, kind="box")
+    rays8[::3, 7] = np.float32(0.4)
+    rays = as_rays(rays8)
+    for mode, ref_order in ((ref.MODE_LOWEST_ID, False), (ref.MODE_VISIT_ORDER, True)):
+        want_b = ref.trace_bvh(nodes, idx, verts, rays, mode=mode, threads=8)
+        want_m = ref.trace_mbvh(quads, idx, verts, rays, mode=mode, threads=8)
+        for tree, want in ((bvh, want_b), (mbvh, want_m)):
+            assert hits_equal(_gpu_hits(tree, verts, rays8, ref_order), want).all(), mode
+            occ = tree.occluded(_dev(verts), _dev(rays8), reference_order=ref_order).cpu().numpy()
+            assert np.array_equal(occ, (want["prim"] != 0xFFFFFFFF).astype(np.uint8)), mode
