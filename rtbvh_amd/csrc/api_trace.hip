@@ -546,7 +546,7 @@ ResultCode autotune(const RTRay* rays, size_t ray_count, RTHit* hits, void* stre
         return hip_fail(e, "autotune events");
     }
     const TraceConfig before = get_trace_config();
-    // compressed tree (one kernel): wave-range schedule with block x LDS
+    // compressed tree (one kernel): rays dealt in runs, with block x LDS
     // depth x grid x refill, and the static schedule at the default shape;
     // 4-wide trees, one-item kernel: block x LDS depth x grid x refill x
     // schedule; per-node-leaves kernel: block x LDS depth x grid

@@ -41,7 +41,7 @@ struct TraceParams {
     uint32_t postpone;     // set by the launcher (compressed tree): triangle tests wait until
                            // this many lanes of the wave have one (0: never wait)
     bool small_leaves;     // every leaf holds at most 16 triangles (one-item kernel)
-    uint32_t wave_ranges;  // set by the launcher: 1 each wave draws from its own ray range
+    uint32_t wave_runs;    // set by the launcher: 1 rays dealt to the waves in runs (RaySchedule)
     const uint32_t* ray_ids;  // non-null (compressed tree, one scene): position j traces ray
                               // ray_ids[j] and writes its result at ray_ids[j]
 };
@@ -57,7 +57,7 @@ struct TraceConfig {
     uint32_t refill;         // one-item kernel: idle lanes of a wave that take new rays
                              // together (1..64)
     uint32_t schedule;       // one-item and compressed kernels: 0 fixed ray stride per lane,
-                             // 1 each wave's lanes draw from the wave's own ray range
+                             // 1 rays dealt to the waves in runs (RaySchedule)
     uint32_t postpone;       // compressed tree: triangle tests wait until this many lanes
                              // of a wave have one, unless a lane has nothing else (0..64)
 };

@@ -349,7 +349,7 @@ __global__ void __launch_bounds__(kBlock) bvh_trace_kernel(TraceParams p) {
         if (takers == 0 && busy == 0) break;  // wave-uniform: no ray left for any lane
         bool take = false;
         if (takers != 0 && (uint32_t(__popcll(takers)) >= refill || busy == 0))
-            take = sched.take(can_take, takers);
+            take = sched.take(p, can_take, takers);
         const uint64_t rid = sched.rid;
         if (take) {
             const bool ok = load_ray(p.rays, rid, s);
@@ -446,7 +446,7 @@ int persistent_grid(K kernel, uint64_t work_items) {
 }
 
 // Grid and hand-out of a RaySchedule kernel: with a few rays per resident
-// lane each wave draws from its own range, refilling 16 lanes at once (half
+// lane the rays are dealt to the waves in runs, refilling 16 lanes at once (half
 // the rays per lane when there are fewer), in up to 8 times the resident
 // blocks; below 2 rays per resident lane, one ray per lane.
 template <typename K>
@@ -454,10 +454,10 @@ int scheduled_grid(K kernel, TraceParams& p) {
     const uint64_t resident = resident_blocks(kernel);
     const uint64_t per_lane = p.ray_count / (resident * kBlock);
     const uint64_t need = (p.ray_count + kBlock - 1) / kBlock;
-    p.wave_ranges = per_lane >= 2 ? 1u : 0u;
+    p.wave_runs = per_lane >= 2 ? 1u : 0u;
     p.refill = per_lane >= 2 ? uint32_t(per_lane / 2 < 16 ? per_lane / 2 : 16) : 1u;
     uint64_t blocks = need;
-    if (p.wave_ranges) {
+    if (p.wave_runs) {
         blocks = need / (p.refill > 8 ? p.refill : 8u);
         blocks = blocks < resident ? resident : (blocks > 8 * resident ? 8 * resident : blocks);
     }

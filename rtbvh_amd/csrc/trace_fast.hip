@@ -381,7 +381,7 @@ __global__ void __launch_bounds__(kMaxBlock) mbvh_item_kernel(TraceParams p) {
         if (takers == 0 && busy == 0) break;  // wave-uniform: no ray left for any lane
         bool take = false;
         if (takers != 0 && (uint32_t(__popcll(takers)) >= refill || busy == 0))
-            take = sched.take(can_take, takers);
+            take = sched.take(p, can_take, takers);
         const uint64_t rid = sched.rid;
         if (take) {
             const float4* r4 = reinterpret_cast<const float4*>(p.rays + rid);
@@ -706,7 +706,7 @@ cw8_kernel(TraceParams p) {
         if (takers == 0 && busy == 0) break;  // wave-uniform: no ray left for any lane
         bool take = false;
         if (takers != 0 && (uint32_t(__popcll(takers)) >= refill || busy == 0))
-            take = sched.take(can_take, takers);
+            take = sched.take(p, can_take, takers);
         const uint64_t rid = sched.rid;
         if (take) {
             if (IDS) cur = p.ray_ids[rid];
@@ -956,16 +956,16 @@ hipError_t launch_fast(const TraceParams& p0, hipStream_t stream) {
     }
     uint64_t blocks = uint64_t(cache_blocks[dev]) * cfg.occupancy_pct / 100;
     if (blocks == 0) blocks = 1;
-    // Wave ranges need a few rays per lane: with r rays per resident lane
-    // they run with refill min(refill, r / 2) and enough waves to fill the
+    // Runs of rays per wave need a few rays per lane: with r rays per resident
+    // lane they go with refill min(refill, r / 2) and enough waves to fill the
     // device, but no more than leave each lane max(refill, 8) rays; launches
     // with fewer than 2 rays per resident lane (a scene of a few thousand
     // triangles) run the static schedule with refill 1.
     const uint64_t resident = uint64_t(cache_blocks[dev]);
     const uint64_t rays_per_lane = p0.ray_count / (resident * cfg.block);
-    const bool ranges = (ITEM || CW8) && cfg.schedule == 1 && rays_per_lane >= 2;
+    const bool runs = (ITEM || CW8) && cfg.schedule == 1 && rays_per_lane >= 2;
     uint32_t refill = cfg.schedule == 1 ? 1u : cfg.refill;
-    if (ranges) {
+    if (runs) {
         refill = uint32_t(rays_per_lane / 2 < cfg.refill ? rays_per_lane / 2 : cfg.refill);
         if (refill == 0) refill = 1;
         const uint64_t per_block = uint64_t(cfg.block) * (refill > 8 ? refill : 8u);
@@ -980,7 +980,7 @@ hipError_t launch_fast(const TraceParams& p0, hipStream_t stream) {
     p.lds_depth = cfg.lds_depth;
     p.refill = refill;
     p.postpone = cfg.postpone;
-    p.wave_ranges = ranges ? 1u : 0u;
+    p.wave_runs = runs ? 1u : 0u;
     hipLaunchKernelGGL(k, dim3(grid), dim3(cfg.block), lds, stream, p);
     return hipGetLastError();
 }
