@@ -379,8 +379,8 @@ ResultCode rtbvh_gpu_adjoint(const float* vertices, size_t prim_count, const RTR
     }
     const hipError_t e = launch_adjoint(
         vertices, uint32_t(prim_count), reinterpret_cast<const DevRay*>(rays),
-        reinterpret_cast<const DevHit*>(hits), ray_count, grad_tuv, grad_vertices, grad_origin,
-        grad_direction, static_cast<hipStream_t>(stream));
+        reinterpret_cast<const DevHit*>(hits), ray_count, grad_tuv, grad_tuv + 1, grad_tuv + 2, 3,
+        grad_vertices, grad_origin, grad_direction, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "adjoint launch");
     return Ok;
 }

@@ -201,7 +201,8 @@ enum WorkspaceKind : int {
     kWsTree = 2,
     kWsSpatial = 3,
     kWsRayOrder = 4,
-    kWsKinds = 5
+    kWsAdjoint = 5,
+    kWsKinds = 6
 };
 constexpr size_t kWorkspaceCacheMax = size_t(1) << 30;
 struct Workspace {
@@ -268,9 +269,12 @@ hipError_t launch_prepare_triangles(const uint32_t* indices, uint32_t index_coun
                                     hipStream_t stream, const uint32_t* scene_off = nullptr,
                                     uint32_t scenes = 0);
 
-// Adjoint of the hit (t, u, v) with respect to vertices and rays (adjoint.hip).
+// Adjoint of the hit (t, u, v) with respect to vertices and rays
+// (adjoint.hip); the gradients of t, u and v are grad_step floats apart, a
+// null one is zero.
 hipError_t launch_adjoint(const float* verts, uint32_t prim_count, const DevRay* rays,
-                          const DevHit* hits, uint64_t ray_count, const float* grad_tuv,
+                          const DevHit* hits, uint64_t ray_count, const float* grad_t,
+                          const float* grad_u, const float* grad_v, uint32_t grad_step,
                           float* grad_verts, float* grad_origin, float* grad_dir,
                           hipStream_t stream);
 

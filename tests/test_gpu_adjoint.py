@@ -25,6 +25,7 @@ from rtbvh_amd import scenes
 
 torch = pytest.importorskip("torch")
 import rtbvh_amd as rt  # noqa: E402
+from rtbvh_amd import diff  # noqa: E402
 from rtbvh_amd.diff import trace_tuv  # noqa: E402
 
 pytestmark = pytest.mark.gpu
@@ -226,3 +227,39 @@ def test_trace_tree_snapshot_guard():
     tree2 = bvh2.trace_tree(verts)
     t2, _, _, _ = trace_tuv(tree2, verts, o, d)
     assert not torch.equal(t, t2)
+
+
+@pytest.mark.parametrize("rays_n, prims", [((1 << 19) - 1, 65), (1 << 19, 64), (1 << 19, 65),
+                                           ((1 << 19) + 4097, 3), ((1 << 19) + 4097, 1000),
+                                           ((1 << 22) + 5, 70_001), (1 << 20, 1_048_577)])
+def test_vertex_gradients_of_many_rays(rays_n, prims):
+    """From 2^19 rays on the vertex terms go through buckets of triangles (64
+    to a bucket up to 65,536 triangles, then 128 and more; above 1,048,576 they
+    go by atomics), tiles of 4096 rays and passes of 2^22.  lambda is dL/d(origin), so the sums have an exact
+    reference: the same float32 terms added in float64.  A float32 sum of k
+    terms is within (k + 2) 2^-24 of it, relative to the sum of magnitudes."""
+    g = torch.Generator("cuda").manual_seed(rays_n + prims)
+    verts = torch.rand((prims, 9), device="cuda", generator=g) * 4.0
+    rays = torch.rand((rays_n, 8), device="cuda", generator=g) + 0.1
+    hits = torch.rand((rays_n, 4), device="cuda", generator=g) * 0.5
+    prim = torch.randint(0, prims, (rays_n,), device="cuda", generator=g, dtype=torch.int32)
+    prim[::7] = -1  # misses
+    hits[:, 3] = prim.view(torch.float32)
+    grad = torch.randn((rays_n, 3), device="cuda", generator=g)
+    d_v, d_o, d_d = diff.adjoint(verts, rays, hits, grad)
+    hit = prim >= 0
+    u, v = hits[hit, 1], hits[hit, 2]
+    lam = d_o[hit]
+    assert not d_o[~hit].any() and not d_d[~hit].any()
+    assert torch.equal(d_d[hit], hits[hit, 0:1] * lam)
+    w = torch.stack([-((1.0 - u) - v), -u, -v], dim=1)
+    terms = (w[:, :, None] * lam[:, None, :]).reshape(-1, 9)
+    idx = prim[hit].long()
+    want = torch.zeros((prims, 9), dtype=torch.float64, device="cuda")
+    size = torch.zeros_like(want)
+    want.index_add_(0, idx, terms.double())
+    size.index_add_(0, idx, terms.double().abs())
+    k = torch.zeros(prims, dtype=torch.float64, device="cuda")
+    k.index_add_(0, idx, torch.ones(len(idx), dtype=torch.float64, device="cuda"))
+    bound = (k[:, None] + 2.0) * 2.0 ** -24 * size
+    assert bool(((d_v.double() - want).abs() <= bound).all())
