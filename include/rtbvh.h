@@ -414,6 +414,20 @@ ResultCode rtbvh_gpu_adjoint(const float *vertices, size_t prim_count, const RTR
                              const RTHit *hits, size_t ray_count, const float *grad_tuv,
                              float *grad_vertices, float *grad_origin, float *grad_direction,
                              void *stream);
+/* The same with the three gradients in arrays of their own (1 float per ray
+ * each); a NULL one is zero. */
+ResultCode rtbvh_gpu_adjoint_parts(const float *vertices, size_t prim_count, const RTRay *rays,
+                                   const RTHit *hits, size_t ray_count, const float *grad_t,
+                                   const float *grad_u, const float *grad_v,
+                                   float *grad_vertices, float *grad_origin,
+                                   float *grad_direction, void *stream);
+/* Ray records from origins and directions (3 floats per ray each) with one
+ * t_min and t_max, and hit records as arrays: t, u, v and the primitive id as
+ * a 64-bit integer, -1 on a miss.  Device pointers; one pass each. */
+ResultCode rtbvh_gpu_pack_rays(const float *origins, const float *directions, size_t ray_count,
+                               float t_min, float t_max, RTRay *rays, void *stream);
+ResultCode rtbvh_gpu_split_hits(const RTHit *hits, size_t ray_count, float *t, float *u, float *v,
+                                int64_t *prim, void *stream);
 
 /* ---- Batches of scenes ---------------------------------------------------
  * Many scenes of uneven size built and traced together (no counterpart in

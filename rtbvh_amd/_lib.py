@@ -117,6 +117,9 @@ SIGNATURES = {
     "rtbvh_gpu_autotune_batch": (_rc, [RTBatch, _vp, _vp, _sz, _vp, _vp,
                                       ctypes.POINTER(RTTraceConfig)]),
     "rtbvh_gpu_adjoint": (_rc, [_vp, _sz, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _vp]),
+    "rtbvh_gpu_adjoint_parts": (_rc, [_vp, _sz, _vp, _vp, _sz, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "rtbvh_gpu_pack_rays": (_rc, [_vp, _vp, _sz, ctypes.c_float, ctypes.c_float, _vp, _vp]),
+    "rtbvh_gpu_split_hits": (_rc, [_vp, _sz, _vp, _vp, _vp, _vp, _vp]),
     "rtbvh_gpu_batch_plan_create": (_rc, [_vp, _vp, _sz, _vp, _vp, _sz, _vp,
                                          ctypes.POINTER(RTBatchPlan)]),
     "rtbvh_gpu_batch_plan_enqueue": (_rc, [RTBatchPlan, _vp, _vp, _vp, _vp, _vp, _sz, _vp, _vp,

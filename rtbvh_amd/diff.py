@@ -1,7 +1,7 @@
 """Differentiable closest hit: a torch.autograd.Function over the C ABI.
 
 Forward: rtbvh_gpu_intersect / rtbvh_gpu_intersect_mbvh (lowest-(t, id)
-rule).  Backward: rtbvh_gpu_adjoint, the analytic adjoint of
+rule).  Backward: rtbvh_gpu_adjoint_parts, the analytic adjoint of
 o + t d = (1-u-v) v0 + u v1 + v v2 with the hit triangle fixed by the
 forward pass (no counterpart in the reference, whose triangle test,
 src/builders/spatial_sah.rs:132-163, is forward only).
@@ -13,7 +13,7 @@ import ctypes
 import torch
 
 from . import _lib as L
-from .api import RAY_FLOATS, TraceTree, _ptr, _require_device, _stream, hits_prim, rays_tensor
+from .api import RAY_FLOATS, TraceTree, _ptr, _require_device, _stream, rays_tensor
 
 
 def adjoint(vertices: torch.Tensor, rays: torch.Tensor, hits: torch.Tensor,
@@ -38,14 +38,39 @@ def adjoint(vertices: torch.Tensor, rays: torch.Tensor, hits: torch.Tensor,
     return gv, go, gd
 
 
+def _pack_rays(origins, directions, t_min, t_max):
+    """rays_tensor in one pass where the library's kernel applies: contiguous
+    (R, 3) float32 arrays on one device and plain numbers for t_min, t_max."""
+    same = (origins.dim() == 2 and origins.shape == directions.shape and origins.shape[1] == 3
+            and origins.dtype == directions.dtype == torch.float32
+            and origins.device.type == "cuda" and origins.device == directions.device
+            and origins.is_contiguous() and directions.is_contiguous())
+    if not same or not all(isinstance(x, (int, float)) for x in (t_min, t_max)):
+        return rays_tensor(origins, directions, t_min, t_max)
+    r = torch.empty((origins.shape[0], RAY_FLOATS), dtype=torch.float32, device=origins.device)
+    L.check(L.lib().rtbvh_gpu_pack_rays(_ptr(origins), _ptr(directions), r.shape[0], float(t_min),
+                                        float(t_max), _ptr(r), _stream(r)), "rtbvh_gpu_pack_rays")
+    return r
+
+
+def _split_hits(hits):
+    """(t, u, v, prim id as int64, -1 on a miss) of (R, 4) hit records."""
+    r = hits.shape[0]
+    t, u, v = (torch.empty(r, dtype=torch.float32, device=hits.device) for _ in range(3))
+    prim = torch.empty(r, dtype=torch.int64, device=hits.device)
+    L.check(L.lib().rtbvh_gpu_split_hits(_ptr(hits), r, _ptr(t), _ptr(u), _ptr(v), _ptr(prim),
+                                         _stream(hits)), "rtbvh_gpu_split_hits")
+    return t, u, v, prim
+
+
 class TraceTUV(torch.autograd.Function):
     """(vertices, origins, directions) -> (t, u, v, prim) of the closest hit."""
 
     @staticmethod
     def forward(ctx, vertices, origins, directions, tree, t_min, t_max):
         verts = vertices.detach().contiguous()
-        rays = rays_tensor(origins.detach().contiguous(), directions.detach().contiguous(),
-                           t_min, t_max)
+        rays = _pack_rays(origins.detach().contiguous(), directions.detach().contiguous(),
+                          t_min, t_max)
         if isinstance(tree, TraceTree):
             # a traversal tree traces its own snapshot of the triangles: the
             # gradients are only those of `vertices` if the snapshot is theirs
@@ -56,21 +81,28 @@ class TraceTUV(torch.autograd.Function):
             hits = tree.intersect(rays)
         else:
             hits = tree.intersect(verts.reshape(-1, 9), rays)
-        prim = hits_prim(hits)
+        t, u, v, prim = _split_hits(hits)
         ctx.save_for_backward(verts, rays, hits)
         ctx.mark_non_differentiable(prim)
-        return hits[:, 0].clone(), hits[:, 1].clone(), hits[:, 2].clone(), prim
+        return t, u, v, prim
 
     @staticmethod
     def backward(ctx, gt, gu, gv, _gprim):
         verts, rays, hits = ctx.saved_tensors
-        r = rays.shape[0]
-        z = torch.zeros(r, dtype=torch.float32, device=rays.device)
-        g = torch.stack([gt if gt is not None else z, gu if gu is not None else z,
-                         gv if gv is not None else z], dim=1).contiguous()
+        parts = [None if g is None else g.contiguous() for g in (gt, gu, gv)]
+        for name, x in (("vertices", verts), ("rays", rays), ("hits", hits),
+                        *((f"grad_{k}", g) for k, g in zip("tuv", parts) if g is not None)):
+            _require_device(x, name)
         need_v = ctx.needs_input_grad[0]
         need_r = ctx.needs_input_grad[1] or ctx.needs_input_grad[2]
-        d_v, d_o, d_d = adjoint(verts.reshape(-1, 9), rays, hits, g, need_v, need_r)
+        n, r = verts.numel() // 9, rays.shape[0]
+        d_v = (torch.zeros((n, 9), dtype=torch.float32, device=verts.device) if need_v else None)
+        d_o, d_d = ((torch.empty((r, 3), dtype=torch.float32, device=rays.device)
+                     for _ in range(2)) if need_r else (None, None))
+        L.check(L.lib().rtbvh_gpu_adjoint_parts(_ptr(verts), n, _ptr(rays), _ptr(hits), r,
+                                                *(_ptr(g) for g in parts), _ptr(d_v), _ptr(d_o),
+                                                _ptr(d_d), _stream(rays)),
+                "rtbvh_gpu_adjoint_parts")
         d_v = d_v.view(verts.shape) if d_v is not None else None
         return (d_v, d_o if ctx.needs_input_grad[1] else None,
                 d_d if ctx.needs_input_grad[2] else None, None, None, None)

@@ -263,3 +263,52 @@ def test_vertex_gradients_of_many_rays(rays_n, prims):
     k.index_add_(0, idx, torch.ones(len(idx), dtype=torch.float64, device="cuda"))
     bound = (k[:, None] + 2.0) * 2.0 ** -24 * size
     assert bool(((d_v.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("n", [0, 1, 255, 257])
+def test_packed_rays_and_split_hits_equal_the_field_copies(n):
+    """One-pass packing and splitting against the per-field forms, with
+    arguments that take the general form (other types, strides, tensors for
+    t_min) beside them."""
+    g = torch.Generator("cuda").manual_seed(n)
+    o = torch.rand((n, 3), device="cuda", generator=g)
+    d = torch.rand((n, 3), device="cuda", generator=g)
+    want = rt.rays_tensor(o, d, 0.25, 7.5)
+    assert torch.equal(diff._pack_rays(o, d, 0.25, 7.5), want)
+    assert torch.equal(diff._pack_rays(o.double(), d, 0.25, 7.5), want)
+    wide = torch.empty((n, 6), device="cuda")
+    wide[:, ::2] = o
+    assert torch.equal(diff._pack_rays(wide[:, ::2], d, 0.25, 7.5), want)
+    t0 = torch.full((n,), 0.25, device="cuda")
+    assert torch.equal(diff._pack_rays(o, d, t0, 7.5), want)
+    hits = torch.rand((n, 4), device="cuda", generator=g)
+    ids = torch.randint(-1, 5, (n,), device="cuda", generator=g, dtype=torch.int32)
+    hits[:, 3] = ids.view(torch.float32)
+    if n > 4:  # an id beyond 2^31
+        hits.view(torch.int32)[3, 3] = -5
+    t, u, v, prim = diff._split_hits(hits)
+    for got, column in ((t, 0), (u, 1), (v, 2)):
+        assert torch.equal(got, hits[:, column])
+    assert prim.dtype == torch.int64 and torch.equal(prim, rt.hits_prim(hits))
+
+
+def test_backward_of_one_output_and_of_expanded_gradients():
+    """Gradients that autograd leaves out are zeros, and a sum's gradient is
+    one number expanded over the rays (stride 0)."""
+    verts = torch.from_numpy(scenes.noisy_sphere(40, 30, seed=3)).cuda().requires_grad_()
+    aabbs, centers = scenes.triangle_aabbs_centers(verts.detach().cpu().numpy())
+    bvh = rt.Builder(torch.from_numpy(centers).cuda(),
+                     aabbs=torch.from_numpy(aabbs).cuda()).construct_locally_ordered_clustered()
+    rays = torch.from_numpy(scenes.rays_sphere_to_box(3000, [0.2] * 3, [0.8] * 3, seed=4)).cuda()
+    o = rays[:, 0:3].contiguous().requires_grad_()
+    d = rays[:, 4:7].contiguous().requires_grad_()
+    t, u, v, prim = trace_tuv(bvh, verts, o, d)
+    assert int((prim >= 0).sum()) > 1000
+    got = torch.autograd.grad(u.sum(), [verts, o, d])
+    hits = torch.stack([t.detach(), u.detach(), v.detach(),
+                        prim.to(torch.int32).view(torch.float32)], dim=1).contiguous()
+    grad = torch.zeros((len(rays), 3), device="cuda")
+    grad[:, 1] = 1.0
+    want = diff.adjoint(verts.detach(), rays, hits, grad)
+    assert torch.allclose(got[0], want[0], rtol=1e-5, atol=1e-5 * float(want[0].abs().max()))
+    assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
