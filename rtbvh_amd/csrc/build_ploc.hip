@@ -63,17 +63,76 @@ struct Bounds6 {
     float mn[3], mx[3];
 };
 
-// half_area(a.union_of(b)) (src/aabb.rs:74-86, 343-346) as a clustering
-// distance.  IEEE min/max give the same values as f32::min/max here: both
-// ignore a NaN operand, and where they differ (the sign of a zero) the
-// resulting distance compares equal.  Stored bounds use rs_min/rs_max.
-__device__ __forceinline__ float dist6(float an0, float an1, float an2, float ax0, float ax1,
-                                       float ax2, float bn0, float bn1, float bn2, float bx0,
-                                       float bx1, float bx2) {
-    const float d0 = fmaxf(ax0, bx0) - fminf(an0, bn0);
-    const float d1 = fmaxf(ax1, bx1) - fminf(an1, bn1);
-    const float d2 = fmaxf(ax2, bx2) - fminf(an2, bn2);
-    return (d0 + d1) * d2 + d0 * d1;
+// v_min_f32 / v_max_f32 themselves: fminf and fmaxf put a canonicalising
+// v_max in front of every operand that comes from memory.
+__device__ __forceinline__ float vmin(float a, float b) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float vmax(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// Nearest neighbour of cluster li of an LDS window of bounds (six arrays,
+// STRIDE apart, minima first): the lowest half_area(a.union_of(b))
+// (src/aabb.rs:74-86, 343-346) over the kRadius positions on either side, the
+// first of equal ones (locb.rs:92-142).  Every position of the window must be
+// readable; those outside the cluster set hold sentinel bounds, whose
+// distance is infinite (put_sentinel).  IEEE min/max give the same values as
+// f32::min/max here: both ignore a NaN operand, and where they differ (the
+// sign of a zero) the resulting distance compares equal.  sc: the scenes of
+// a batch (null: one scene).  Returns the offset, 0 when there is none.
+//
+// Unrolled with fixed offsets, so that a candidate costs six LDS reads at
+// immediate addresses and 16 VALU (26 with bounds checks and fminf / fmaxf),
+// in four chains of comparisons that join in order.  1M triangles: the tail
+// kernel 741 -> 551 us, the 59 neighbour searches 514 -> 372 us per build.
+template <int STRIDE, bool SEG, typename SC>
+__device__ __forceinline__ int nearest_offset(const float* b, uint32_t li, const SC* sc) {
+    const float* w = b + li;
+    const float an0 = w[0], an1 = w[STRIDE], an2 = w[2 * STRIDE];
+    const float ax0 = w[3 * STRIDE], ax1 = w[4 * STRIDE], ax2 = w[5 * STRIDE];
+    constexpr int kChain = 4, kEach = 2 * kRadius / kChain;
+    static_assert(kChain * kEach == 2 * kRadius, "equal chains");
+    float best[kChain];
+    int off[kChain];
+#pragma unroll
+    for (int c = 0; c < kChain; ++c) {
+        best[c] = 3.40282347e38f;  // f32::MAX (locb.rs:95)
+        off[c] = 0;
+    }
+#pragma unroll
+    for (int q = 0; q < kEach; ++q)
+#pragma unroll
+        for (int c = 0; c < kChain; ++c) {
+            const int k = c * kEach + q;
+            const int o = k < kRadius ? k - kRadius : k - kRadius + 1;
+            const float d0 = vmax(ax0, w[o + 3 * STRIDE]) - vmin(an0, w[o]);
+            const float d1 = vmax(ax1, w[o + 4 * STRIDE]) - vmin(an1, w[o + STRIDE]);
+            const float d2 = vmax(ax2, w[o + 5 * STRIDE]) - vmin(an2, w[o + 2 * STRIDE]);
+            const float d = (d0 + d1) * d2 + d0 * d1;
+            bool nearer = d < best[c];
+            if (SEG) nearer = nearer & (sc[int(li) + o] == sc[li]);
+            best[c] = nearer ? d : best[c];
+            off[c] = nearer ? o : off[c];
+        }
+    for (int c = 1; c < kChain; ++c)
+        if (best[c] < best[0]) {
+            best[0] = best[c];
+            off[0] = off[c];
+        }
+    return off[0];
+}
+
+template <int STRIDE>
+__device__ __forceinline__ void put_sentinel(float* b, uint32_t li) {
+    for (int k = 0; k < 3; ++k) {
+        b[k * STRIDE + li] = -__builtin_inff();
+        b[(3 + k) * STRIDE + li] = __builtin_inff();
+    }
 }
 
 __device__ __forceinline__ Bounds6 bounds_of(const DevAabb& a) {
@@ -462,19 +521,11 @@ struct PlocState {
     uint32_t pad[2];
 };
 
-__device__ __forceinline__ void nn_window(uint32_t i, uint32_t n, uint32_t& sb, uint32_t& se) {
-    // search_range, locb.rs:36-45 (relative to begin = 0)
-    sb = i > uint32_t(kRadius) ? i - kRadius : 0u;
-    se = (i + kRadius + 1) < n ? i + kRadius + 1 : n;
-}
-
 // Nearest neighbour + mutual marks for one tile.  Bounds are staged in LDS
 // as six arrays so that lanes reading consecutive clusters hit consecutive
 // banks.  kNnBlock threads cover the tile and its halo (kTile + 2 kRadius
-// neighbour searches) in one pass, and each search loads its candidates four
-// at a time and compares them in index order (the first lowest distance
-// wins, as in the sequential loop): later iterations are short, and their
-// time is the latency of this chain.
+// neighbour searches) in one pass: later iterations are short, and their time
+// is the latency of the search (nearest_offset).
 constexpr int kNnBlock = 320;
 static_assert(kNnBlock >= kTile + 2 * kRadius, "one neighbour search per thread");
 static_assert(kNnBlock >= kTile + 4 * kRadius, "staging in one pass");
@@ -498,52 +549,29 @@ __global__ void __launch_bounds__(kNnBlock)
     const uint32_t ts = blockIdx.x * kTile;
     if (ts >= n) return;
     const uint32_t te = ts + kTile < n ? ts + kTile : n;
-    const uint32_t lb = ts > uint32_t(kHalo) ? ts - kHalo : 0u;
-    const uint32_t le = te + kHalo < n ? te + kHalo : n;
     if (threadIdx.x == 0) s_total = 0;
-    for (uint32_t k = lb + threadIdx.x; k < le; k += kNnBlock) {
-        DevAabb a;
-        load_node(cl + k, a);
-        s_b[0][k - lb] = a.min[0];
-        s_b[1][k - lb] = a.min[1];
-        s_b[2][k - lb] = a.min[2];
-        s_b[3][k - lb] = a.max[0];
-        s_b[4][k - lb] = a.max[1];
-        s_b[5][k - lb] = a.max[2];
-        if (SEG) s_sc[k - lb] = cs[k];
+    // window position k holds cluster ts - kHalo + k, or a sentinel
+    for (uint32_t k = threadIdx.x; k < uint32_t(kSpan); k += kNnBlock) {
+        const uint32_t i = ts + k - kHalo;  // wraps below 0, to above n
+        if (i < n) {
+            DevAabb a;
+            load_node(cl + i, a);
+            for (int c = 0; c < 3; ++c) {
+                s_b[c][k] = a.min[c];
+                s_b[3 + c][k] = a.max[c];
+            }
+            if (SEG) s_sc[k] = cs[i];
+        } else {
+            put_sentinel<kSpan>(&s_b[0][0], k);
+            if (SEG) s_sc[k] = 0xFFFFFFFFu;
+        }
     }
     __syncthreads();
     const uint32_t nb0 = ts > uint32_t(kRadius) ? ts - kRadius : 0u;
     const uint32_t nb1 = te + kRadius < n ? te + kRadius : n;
     for (uint32_t i = nb0 + threadIdx.x; i < nb1; i += kNnBlock) {
-        uint32_t s0, s1;
-        nn_window(i, n, s0, s1);
-        const uint32_t li = i - lb;
-        const float a0 = s_b[0][li], a1 = s_b[1][li], a2 = s_b[2][li];
-        const float a3 = s_b[3][li], a4 = s_b[4][li], a5 = s_b[5][li];
-        float best = 3.40282347e38f;  // f32::MAX (locb.rs:95)
-        uint32_t best_j = 0xFFFFFFFFu;
-        for (uint32_t j0 = s0; j0 < s1; j0 += 4) {
-            float d[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const uint32_t j = j0 + uint32_t(u);
-                // a position past the window reads a staged cluster and is
-                // dropped (NaN never compares less)
-                const uint32_t lj = (j < s1 ? j : s1 - 1) - lb;
-                const bool skip = j >= s1 || j == i || (SEG && s_sc[lj] != s_sc[li]);
-                const float dd = dist6(a0, a1, a2, a3, a4, a5, s_b[0][lj], s_b[1][lj],
-                                       s_b[2][lj], s_b[3][lj], s_b[4][lj], s_b[5][lj]);
-                d[u] = skip ? __builtin_nanf("") : dd;
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (d[u] < best) {
-                    best = d[u];
-                    best_j = j0 + uint32_t(u);
-                }
-        }
-        s_nb[i - nb0] = best_j;
+        const int o = nearest_offset<kSpan, SEG>(&s_b[0][0], i + kHalo - ts, s_sc);
+        s_nb[i - nb0] = o ? i + uint32_t(o) : 0xFFFFFFFFu;
     }
     __syncthreads();
     uint32_t cnt = 0;
@@ -682,24 +710,24 @@ constexpr int kTailWaves = kTailThreads / 64;
 template <bool SEG, int CAP>
 struct TailShared {
     static constexpr int kPer = CAP / kTailThreads;  // clusters per thread
-    float b[6][CAP];
+    // kRadius sentinels before the clusters and after the last
+    static constexpr int kStride = CAP + 2 * kRadius;
+    float b[6][kStride];
     int32_t e1[CAP];
     int32_t e2[CAP];
     uint16_t nb[CAP];
     uint16_t m[CAP];
-    uint16_t sc[SEG ? CAP : 2];  // scene of each cluster (batches)
+    uint16_t sc[SEG ? kStride : 2];  // scene of each cluster (batches), placed as b
     uint32_t wsum[kPer * kTailWaves];
 };
 
 template <typename TS>
 __device__ __forceinline__ DevAabb tail_node(const TS& sh, uint32_t i) {
     DevAabb a;
-    a.min[0] = sh.b[0][i];
-    a.min[1] = sh.b[1][i];
-    a.min[2] = sh.b[2][i];
-    a.max[0] = sh.b[3][i];
-    a.max[1] = sh.b[4][i];
-    a.max[2] = sh.b[5][i];
+    for (int c = 0; c < 3; ++c) {
+        a.min[c] = sh.b[c][kRadius + i];
+        a.max[c] = sh.b[3 + c][kRadius + i];
+    }
     a.extra1 = sh.e1[i];
     a.extra2 = sh.e2[i];
     return a;
@@ -707,12 +735,10 @@ __device__ __forceinline__ DevAabb tail_node(const TS& sh, uint32_t i) {
 
 template <typename TS>
 __device__ __forceinline__ void tail_store(TS& sh, uint32_t i, const DevAabb& a) {
-    sh.b[0][i] = a.min[0];
-    sh.b[1][i] = a.min[1];
-    sh.b[2][i] = a.min[2];
-    sh.b[3][i] = a.max[0];
-    sh.b[4][i] = a.max[1];
-    sh.b[5][i] = a.max[2];
+    for (int c = 0; c < 3; ++c) {
+        sh.b[c][kRadius + i] = a.min[c];
+        sh.b[3 + c][kRadius + i] = a.max[c];
+    }
     sh.e1[i] = a.extra1;
     sh.e2[i] = a.extra2;
 }
@@ -745,46 +771,26 @@ __global__ void __launch_bounds__(kTailThreads)
         DevAabb a;
         load_node(cl_in + i, a);
         tail_store(sh, i, a);
-        if (SEG) sh.sc[i] = uint16_t(cs_in[i]);
+        if (SEG) sh.sc[kRadius + i] = uint16_t(cs_in[i]);
     }
-    __syncthreads();
+    if (tid < uint32_t(kRadius)) {
+        put_sentinel<TS::kStride>(&sh.b[0][0], tid);
+        if (SEG) sh.sc[tid] = 0;
+    }
     while (n > n_final) {
-        // nearest neighbours
-#pragma unroll
+        // the sentinels after the last cluster
+        if (tid < uint32_t(kRadius)) {
+            put_sentinel<TS::kStride>(&sh.b[0][0], kRadius + n + tid);
+            if (SEG) sh.sc[kRadius + n + tid] = 0;
+        }
+        __syncthreads();
+        // nearest neighbours (one search's registers at a time)
+#pragma unroll 1
         for (int k = 0; k < kTailPer; ++k) {
             const uint32_t i = tid + uint32_t(k) * kTailThreads;
             if (i >= n) continue;
-            uint32_t s0, s1;
-            nn_window(i, n, s0, s1);
-            const float a0 = sh.b[0][i], a1 = sh.b[1][i], a2 = sh.b[2][i];
-            const float a3 = sh.b[3][i], a4 = sh.b[4][i], a5 = sh.b[5][i];
-            const uint32_t si = SEG ? sh.sc[i] : 0u;
-            float best = 3.40282347e38f;
-            uint32_t best_j = 0xFFFFu;
-            // four candidates in flight, compared in index order (as
-            // nn_mark_kernel), where registers allow: the batch instances
-            // (scene ids, or 4096 clusters) would spill, and keep the
-            // one-at-a-time loop
-            constexpr uint32_t kStep = (!SEG && CAP <= int(kTailEnter)) ? 4u : 1u;
-            for (uint32_t j0 = s0; j0 < s1; j0 += kStep) {
-                float d[kStep];
-#pragma unroll
-                for (int u = 0; u < int(kStep); ++u) {
-                    const uint32_t j = j0 + uint32_t(u);
-                    const uint32_t jc = j < s1 ? j : s1 - 1;
-                    const bool skip = j >= s1 || j == i || (SEG && sh.sc[jc] != si);
-                    const float dd = dist6(a0, a1, a2, a3, a4, a5, sh.b[0][jc], sh.b[1][jc],
-                                           sh.b[2][jc], sh.b[3][jc], sh.b[4][jc], sh.b[5][jc]);
-                    d[u] = skip ? __builtin_nanf("") : dd;
-                }
-#pragma unroll
-                for (int u = 0; u < int(kStep); ++u)
-                    if (d[u] < best) {
-                        best = d[u];
-                        best_j = j0 + uint32_t(u);
-                    }
-            }
-            sh.nb[i] = uint16_t(best_j);
+            const int o = nearest_offset<TS::kStride, SEG>(&sh.b[0][0], kRadius + i, sh.sc);
+            sh.nb[i] = uint16_t(o ? i + uint32_t(o) : 0xFFFFu);
         }
         __syncthreads();
         // mutual marks at the lower index and their inclusive prefix
@@ -828,7 +834,7 @@ __global__ void __launch_bounds__(kTailThreads)
             const uint32_t i = tid + uint32_t(k) * kTailThreads;
             dst[k] = 0xFFFFFFFFu;
             if (i >= n) continue;
-            keep_sc[k] = SEG ? sh.sc[i] : uint16_t(0);
+            keep_sc[k] = SEG ? sh.sc[kRadius + i] : uint16_t(0);
             const uint32_t j = sh.nb[i];
             const bool mutual = j < n && sh.nb[j] == i;
             const uint32_t mi = sh.m[i];
@@ -855,12 +861,12 @@ __global__ void __launch_bounds__(kTailThreads)
         for (int k = 0; k < kTailPer; ++k)
             if (dst[k] != 0xFFFFFFFFu) {
                 tail_store(sh, dst[k], keep[k]);
-                if (SEG) sh.sc[dst[k]] = keep_sc[k];
+                if (SEG) sh.sc[kRadius + dst[k]] = keep_sc[k];
             }
-        __syncthreads();
         n -= merged;
         end -= 2 * merged;
     }
+    __syncthreads();
     if (n == n_final)
         for (uint32_t i = tid; i < n; i += kTailThreads) store_node(nodes + i, tail_node(sh, i));
     if (tid == 0) {

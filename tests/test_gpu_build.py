@@ -460,3 +460,18 @@ def test_trace_tree8_duplicates_and_degenerates():
     assert np.array_equal(m.intersect(dv, dr).cpu().numpy().view(ref.HIT).reshape(-1)["prim"],
                           want["prim"])
     assert (want["prim"] != 0xFFFFFFFF).sum() > len(rays8) // 20
+
+
+@pytest.mark.parametrize("n", [3, 14, 15, 28, 29, 30, 255, 256, 257, 284, 2047, 2048, 2049, 2304,
+                               2320, 5000])
+def test_ploc_search_windows_at_tile_edges(n):
+    """The neighbour search reads 14 clusters on either side at fixed
+    offsets: sets smaller than the window, ends of tiles of 256 and of the
+    2048 the last kernel takes, and equal boxes (the first of equal
+    distances)."""
+    verts = scenes.random_soup(n, 0.05, seed=n)
+    verts[1::3] = verts[0]  # equal boxes and Morton codes
+    bvh, aabbs, centers = _build(verts, "ploc")
+    nodes, idx = ref.build_locb(aabbs, centers)
+    assert np.array_equal(_indices(bvh), idx)
+    assert np.array_equal(flat(_nodes(bvh)).view(np.uint32), flat(nodes).view(np.uint32))
