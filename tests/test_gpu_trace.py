@@ -312,3 +312,36 @@ def test_vertex_traversals_over_ray_counts_and_leaf_sizes(rays_n, per_leaf):
             assert hits_equal(_gpu_hits(tree, verts, rays8, ref_order), want).all(), mode
             occ = tree.occluded(_dev(verts), _dev(rays8), reference_order=ref_order).cpu().numpy()
             assert np.array_equal(occ, (want["prim"] != 0xFFFFFFFF).astype(np.uint8)), mode
+
+
+@pytest.mark.parametrize("rays_n", [1, 7, 9, 31, 33, 4097, 98_304, 98_305, 300_001])
+def test_compressed_tree_over_ray_counts(rays_n):
+    """Up to 98,304 rays eight lanes hold a ray and test a node's triangles
+    at once, above a lane holds one: both equal brute force, for one tree, a
+    batch and in any launch shape, with zero direction components, short t_max
+    and duplicated triangles (the lowest id of equal t)."""
+    verts = np.concatenate([scenes.random_soup(300, 0.25, seed=31)] * 2)
+    aabbs, centers = prep(verts)
+    dv, dc, da = _dev(verts), _dev(centers), _dev(flat(aabbs))
+    tree = rt.Builder(dc, aabbs=da).construct_locally_ordered_clustered().trace_tree(dv)
+    rays8 = ray_set(verts, rays_n, seed=rays_n, kind="box")
+    rays8[::5, 4] = 0.0
+    rays8[::11, 5] = 0.0
+    rays8[::3, 7] = np.float32(0.3)
+    want = ref.trace_brute(verts, as_rays(rays8), threads=8)
+    flags = (want["prim"] != 0xFFFFFFFF).astype(np.uint8)
+    dr = _dev(rays8)
+    batch = rt.SceneBatch(dc, [0, len(verts)], aabbs=da)
+    batch.attach_triangles(dv)
+    off = rt.SceneBatch.ray_offsets([rays_n], "cuda")
+    try:
+        for shape in (None, (64, 0, 100, 0, 1, 0), (128, 8, 1600, 0, 16, 1)):
+            rt.set_trace_config(None) if shape is None else rt.set_trace_config(*shape)
+            for got in (tree.intersect(dr), batch.intersect(dr, off),
+                        tree.intersect(dr, order_rays=True)):
+                assert hits_equal(got.cpu().numpy().view(ref.HIT).reshape(-1), want).all(), shape
+            for got in (tree.occluded(dr), batch.occluded(dr, off)):
+                assert np.array_equal(got.cpu().numpy(), flags), shape
+    finally:
+        rt.set_trace_config(None)
+    tree.status()
