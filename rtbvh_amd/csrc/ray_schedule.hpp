@@ -75,6 +75,12 @@ struct RaySchedule {
         return true;
     }
 
+    // Called by the whole wave: no lane will take another ray once those in
+    // hand (`active`) are done, given that none can now.
+    __device__ bool last(const TraceParams& p, bool active) const {
+        return runs || __ballot(active && rid + stride < p.ray_count) == 0;
+    }
+
     // The lane's ray is finished (or skipped).
     __device__ void next() {
         if (!runs) rid += stride;

@@ -662,6 +662,129 @@ __device__ __forceinline__ float qbyte(uint32_t w, int i) {
     return float((w >> ((i & 3) * 8)) & 0xFFu);
 }
 
+// Minimum over the 8 lanes of a group, in every lane.
+template <int CTRL>
+__device__ __forceinline__ float dpp_lane(float x) {
+    return __uint_as_float(uint32_t(
+        __builtin_amdgcn_update_dpp(0, int(__float_as_uint(x)), CTRL, 0xF, 0xF, true)));
+}
+__device__ __forceinline__ float min8(float x) {
+    x = fminf(x, dpp_lane<0xB1>(x));   // quad_perm: the lane's pair
+    x = fminf(x, dpp_lane<0x4E>(x));   // quad_perm: the other pair
+    return fminf(x, dpp_lane<0x141>(x));  // row_half_mirror: the other quad
+}
+
+// A ray held by a group of eight lanes, each with a copy of it.
+struct GroupRay {
+    float ox, oy, oz, dx, dy, dz, ix, iy, iz, tmin;
+    float bt, bu, bv;
+    uint32_t bp;
+};
+
+// Node idx against the ray, a slot per lane: its interior hits become the
+// node group in hand, its triangle hits (ngy and tgy stay 0 without any) the
+// triangle group.  The slot test is cw8_kernel's.
+template <bool ANY>
+__device__ __forceinline__ void group_node(const TraceParams& p, const GroupRay& r, uint32_t idx,
+                                           uint32_t lane8, uint32_t oct, uint32_t& ngx,
+                                           uint32_t& ngy, uint32_t& tgx, uint32_t& tgy) {
+    const uint4* q = reinterpret_cast<const uint4*>(p.cnodes + idx);
+    const uint8_t* planes = reinterpret_cast<const uint8_t*>(q + 2) + lane8;
+    // this lane's slot: near planes first along a positive direction
+    const uint32_t nx = (oct & 1u) ? 24u : 0u, ny = (oct & 2u) ? 32u : 8u,
+                   nz = (oct & 4u) ? 40u : 16u;
+    const uint32_t fx = 24u - nx, fy = 40u - ny, fz = 56u - nz;
+    const uint4 h0 = q[0], h1 = q[1];
+    const float qnx = float(planes[nx]), qfx = float(planes[fx]);
+    const float qny = float(planes[ny]), qfy = float(planes[fy]);
+    const float qnz = float(planes[nz]), qfz = float(planes[fz]);
+    const float stx = __uint_as_float((h0.w & 0xFFu) << 23);
+    const float sty = __uint_as_float(((h0.w >> 8) & 0xFFu) << 23);
+    const float stz = __uint_as_float(((h0.w >> 16) & 0xFFu) << 23);
+    float sx = stx * r.ix, sy = sty * r.iy, sz = stz * r.iz;
+    float bx = (__uint_as_float(h0.x) - r.ox) * r.ix;
+    float by = (__uint_as_float(h0.y) - r.oy) * r.iy;
+    float bz = (__uint_as_float(h0.z) - r.oz) * r.iz;
+    if (oct >= 8u) {
+        if (oct & 8u) {
+            sx = kFlatScale;
+            bx = flat_offset((r.ox - __uint_as_float(h0.x)) / stx);
+        }
+        if (oct & 16u) {
+            sy = kFlatScale;
+            by = flat_offset((r.oy - __uint_as_float(h0.y)) / sty);
+        }
+        if (oct & 32u) {
+            sz = kFlatScale;
+            bz = flat_offset((r.oz - __uint_as_float(h0.z)) / stz);
+        }
+    }
+    const float ex = fmaf(fabsf(sx), 255.0f, fabsf(bx)) * kBoxEps;
+    const float ey = fmaf(fabsf(sy), 255.0f, fabsf(by)) * kBoxEps;
+    const float ez = fmaf(fabsf(sz), 255.0f, fabsf(bz)) * kBoxEps;
+    const float tnx = fmaf(qnx, sx, bx - ex), tfx = fmaf(qfx, sx, bx + ex);
+    const float tny = fmaf(qny, sy, by - ey), tfy = fmaf(qfy, sy, by + ey);
+    const float tnz = fmaf(qnz, sz, bz - ez), tfz = fmaf(qfz, sz, bz + ez);
+    const float en = fmaxf(fmaxf(fmaxf(tnx, tny), tnz), r.tmin);
+    const bool hit = en <= fminf(fminf(fminf(tfx, tfy), tfz), r.bt);
+    const uint32_t hm = uint32_t(__ballot(hit) >> (threadIdx.x & 56u)) & 0xFFu;
+    const uint32_t imask = h0.w >> 24, lmask = h1.z & 0xFFu;
+    const uint32_t ih = hm & imask, th = hm & lmask;
+    const float gmin = min8(hit ? en : 3.0e38f);
+    if (ih) {
+        ngx = h1.x;
+        ngy = (oct_permute(ih, oct) << 24) | (imask << 16) | bound_bits(gmin);
+    }
+    if (th) {
+        tgx = h1.y;
+        tgy = (lmask << 8) | th;
+    }
+}
+
+// Every triangle hit of a triangle group (cw8_kernel's entry) at once, one
+// per lane of its slot; true when any hit is found.
+template <bool ANY>
+__device__ __forceinline__ bool group_triangles(const TraceParams& p, GroupRay& r, uint32_t lane8,
+                                                uint32_t tgx, uint32_t tgy) {
+    MtResult m;
+    m.ok = false;
+    m.t = m.u = m.v = 0.f;
+    uint32_t prim = RTBVH_MISS;
+    if ((tgy >> lane8) & 1u) {
+        const uint32_t pos = tgx + uint32_t(__popc((tgy >> 8) & ((1u << lane8) - 1u)));
+        if (pos < p.index_count) {
+            m = mt_prepared(p.tris, pos, r.ox, r.oy, r.oz, r.dx, r.dy, r.dz, r.tmin, &prim);
+            m.ok = m.ok && prim != RTBVH_MISS &&
+                   (ANY ? m.t < r.bt : lowest_first(m.t, prim, r.bt, r.bp));
+        }
+    }
+    if ((uint32_t(__ballot(m.ok) >> (threadIdx.x & 56u)) & 0xFFu) == 0u) return false;
+    if (ANY) {
+        r.bp = 0;  // any id but RTBVH_MISS
+        return true;
+    }
+    // the lowest (t, id) of the group
+    float t = m.ok ? m.t : __builtin_inff();
+    uint32_t id = m.ok ? prim : RTBVH_MISS;
+    uint32_t who = lane8;
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) {
+        const float ot = __shfl_xor(t, o, 8);
+        const uint32_t oid = __shfl_xor(id, o, 8);
+        const uint32_t ow = __shfl_xor(who, o, 8);
+        if (ot < t || (ot == t && oid < id)) {
+            t = ot;
+            id = oid;
+            who = ow;
+        }
+    }
+    r.bt = t;
+    r.bp = id;
+    r.bu = __shfl(m.u, int(who), 8);
+    r.bv = __shfl(m.v, int(who), 8);
+    return false;
+}
+
 template <bool ANY, bool STATS, bool BATCH, bool IDS = false>
 __global__ void __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(8)))
 cw8_kernel(TraceParams p) {
@@ -687,6 +810,7 @@ cw8_kernel(TraceParams p) {
     uint32_t tgx = 0, tgy = 0;  // triangle group in hand
     bool active = false;
     uint32_t cur = 0;  // IDS: the caller's index of the ray in hand
+    uint64_t group_busy = 0;
     const auto push = [&](uint32_t x, uint32_t y) -> bool {
         if (sp < ldepth) {
             lds_put(lbase + uint32_t(sp) * lstep, x, y);
@@ -704,6 +828,12 @@ cw8_kernel(TraceParams p) {
         const uint64_t takers = __ballot(can_take);
         const uint64_t busy = __ballot(active);
         if (takers == 0 && busy == 0) break;  // wave-uniform: no ray left for any lane
+        // the wave's last rays: a group of eight lanes takes each (below)
+        if (!STATS && takers == 0 && __popcll(busy) <= 8 && sched.last(p, active) &&
+            __ballot(active && sp > ldepth) == 0) {
+            group_busy = busy;
+            break;
+        }
         bool take = false;
         if (takers != 0 && (uint32_t(__popcll(takers)) >= refill || busy == 0))
             take = sched.take(p, can_take, takers);
@@ -913,6 +1043,95 @@ cw8_kernel(TraceParams p) {
             sched.next();
         }
     }
+    if (!STATS && group_busy != 0) {
+        // At most eight rays are left in the wave, and a ray that is long
+        // after 64 others were not may visit thousands of nodes (a camera ray
+        // along a sphere's pole).  2^20 / 2^22 camera rays on 1M triangles 1780 -> 690 /
+        // 1350 -> 1232 us, 2^20 rays uniform in the box of 300k triangles 487 -> 440 us; 2^26
+        // bounce rays unchanged (28.2 ms).  Group g of eight lanes takes the g-th of
+        // them over: its state by shuffles, its stack in its lane's LDS (the
+        // entries beyond go to private arrays, unused so far).
+        const uint32_t lane8 = threadIdx.x & 7u, group = (threadIdx.x >> 3) & 7u;
+        uint64_t rest = group_busy;
+        for (uint32_t k = 0; k < group; ++k) rest &= rest - 1;
+        const int own = rest ? __builtin_ctzll(rest) : 0;
+        GroupRay r;
+        r.ox = __shfl(ox, own, 64);
+        r.oy = __shfl(oy, own, 64);
+        r.oz = __shfl(oz, own, 64);
+        r.dx = __shfl(dx, own, 64);
+        r.dy = __shfl(dy, own, 64);
+        r.dz = __shfl(dz, own, 64);
+        r.ix = __shfl(ix, own, 64);
+        r.iy = __shfl(iy, own, 64);
+        r.iz = __shfl(iz, own, 64);
+        r.tmin = __shfl(tmin, own, 64);
+        r.bt = __shfl(bt, own, 64);
+        r.bu = __shfl(bu, own, 64);
+        r.bv = __shfl(bv, own, 64);
+        r.bp = __shfl(bp, own, 64);
+        oct = __shfl(oct, own, 64);
+        ngx = __shfl(ngx, own, 64);
+        ngy = __shfl(ngy, own, 64);
+        tgx = __shfl(tgx, own, 64);
+        tgy = __shfl(tgy, own, 64);
+        sp = __shfl(sp, own, 64);
+        const uint64_t at = IDS ? uint64_t(__shfl(cur, own, 64))
+                                : (uint64_t(__shfl(uint32_t(sched.rid >> 32), own, 64)) << 32) |
+                                      __shfl(uint32_t(sched.rid), own, 64);
+        const uint32_t gbase = uint32_t(__shfl(int(lbase), own, 64));
+        if (rest == 0) return;  // whole groups; no wave-wide step follows
+        bool overflow = false, found = false;
+        for (;;) {
+            if ((tgy & 0xFFu) != 0u) {
+                found = group_triangles<ANY>(p, r, lane8, tgx, tgy);
+                tgy = 0;
+                if (found) break;
+            }
+            if (ngy >= kNodeGroup && group_bound(ngy) > r.bt) ngy = 0;
+            while (ngy < kNodeGroup && (tgy & 0xFFu) == 0u && sp > 0) {
+                --sp;
+                const uint2 g =
+                    sp < ldepth ? lds_get(gbase + uint32_t(sp) * lstep) : deep[sp - ldepth];
+                if (g.y < kNodeGroup) {
+                    tgx = g.x;
+                    tgy = g.y;
+                } else if (group_bound(g.y) <= r.bt) {
+                    ngx = g.x;
+                    ngy = g.y;
+                }
+            }
+            if (ngy >= kNodeGroup) {
+                const uint32_t key = uint32_t(__builtin_ctz(ngy >> 24));
+                ngy &= ~(1u << (24 + key));
+                const uint32_t slot = key ^ (oct & 7u);
+                const uint32_t idx = ngx + uint32_t(__popc((ngy >> 16) & ((1u << slot) - 1u)));
+                if (ngy >= kNodeGroup) {
+                    if (sp < ldepth)
+                        lds_put(gbase + uint32_t(sp) * lstep, ngx, ngy);
+                    else if (sp < RTBVH_MAX_STACK)
+                        deep[sp - ldepth] = make_uint2(ngx, ngy);
+                    else
+                        overflow = true;
+                    if (overflow) break;
+                    ++sp;
+                }
+                ngy = 0;
+                if (idx < p.node_count)
+                    group_node<ANY>(p, r, idx, lane8, oct, ngx, ngy, tgx, tgy);
+            }
+            if (ngy < kNodeGroup && (tgy & 0xFFu) == 0u && sp == 0) break;
+        }
+        if (lane8 != 0) return;
+        if (overflow) atomicOr(p.status, kStatusStackOverflow);
+        if (ANY) {
+            p.occluded[at] = (r.bp != RTBVH_MISS) ? 1 : 0;
+        } else {
+            store_hit(p.hits, at, overflow ? __builtin_nanf("") : r.bt, r.bu, r.bv,
+                      overflow ? RTBVH_MISS : r.bp);
+        }
+        return;
+    }
     if (STATS) {
         atomicAdd(reinterpret_cast<unsigned long long*>(p.stats), (unsigned long long)n_nodes);
         atomicAdd(reinterpret_cast<unsigned long long*>(p.stats) + 1, (unsigned long long)n_tris);
@@ -940,18 +1159,6 @@ constexpr int kGroupBlock = 256;
 // 1M triangles), at 2^18 more (186 / 179 / 655 against 120 / 168 / 527).
 constexpr uint64_t kGroupRays = 3u << 15;
 
-// Minimum over the 8 lanes of a group, in every lane.
-template <int CTRL>
-__device__ __forceinline__ float dpp_lane(float x) {
-    return __uint_as_float(uint32_t(
-        __builtin_amdgcn_update_dpp(0, int(__float_as_uint(x)), CTRL, 0xF, 0xF, true)));
-}
-__device__ __forceinline__ float min8(float x) {
-    x = fminf(x, dpp_lane<0xB1>(x));   // quad_perm: the lane's pair
-    x = fminf(x, dpp_lane<0x4E>(x));   // quad_perm: the other pair
-    return fminf(x, dpp_lane<0x141>(x));  // row_half_mirror: the other quad
-}
-
 template <bool ANY, bool BATCH>
 __global__ void __launch_bounds__(kGroupBlock) cw8_group_kernel(TraceParams p) {
     if (p.gate && *p.gate) return;  // the tree this launch would read is incomplete
@@ -962,10 +1169,7 @@ __global__ void __launch_bounds__(kGroupBlock) cw8_group_kernel(TraceParams p) {
     int sp = 0;
     const uint64_t stride = uint64_t(gridDim.x) * (kGroupBlock / 8);
     uint64_t rid = uint64_t(blockIdx.x) * (kGroupBlock / 8) + (threadIdx.x >> 3);
-    float ox = 0.f, oy = 0.f, oz = 0.f, dx = 0.f, dy = 0.f, dz = 0.f, ix = 0.f, iy = 0.f,
-          iz = 0.f, tmin = 0.f;
-    float bt = 0.f, bu = 0.f, bv = 0.f;
-    uint32_t bp = RTBVH_MISS;
+    GroupRay ray{};
     uint32_t oct = 0;           // bits 0..2 direction signs, 3..5 axes whose 1/d is infinite
     uint32_t ngx = 0, ngy = 0;  // node group in hand
     bool active = false;
@@ -975,39 +1179,39 @@ __global__ void __launch_bounds__(kGroupBlock) cw8_group_kernel(TraceParams p) {
             const float4* r4 = reinterpret_cast<const float4*>(p.rays + rid);
             const float4 ra = r4[0];
             const float4 rb = r4[1];
-            ox = ra.x;
-            oy = ra.y;
-            oz = ra.z;
-            tmin = ra.w;
-            dx = rb.x;
-            dy = rb.y;
-            dz = rb.z;
-            bt = rb.w;
-            ix = box_inv(dx);
-            iy = box_inv(dy);
-            iz = box_inv(dz);
-            bu = 0.f;
-            bv = 0.f;
-            bp = RTBVH_MISS;
-            const bool nan = (ox != ox) || (oy != oy) || (oz != oz) || (dx != dx) ||
-                             (dy != dy) || (dz != dz);
+            ray.ox = ra.x;
+            ray.oy = ra.y;
+            ray.oz = ra.z;
+            ray.tmin = ra.w;
+            ray.dx = rb.x;
+            ray.dy = rb.y;
+            ray.dz = rb.z;
+            ray.bt = rb.w;
+            ray.ix = box_inv(ray.dx);
+            ray.iy = box_inv(ray.dy);
+            ray.iz = box_inv(ray.dz);
+            ray.bu = 0.f;
+            ray.bv = 0.f;
+            ray.bp = RTBVH_MISS;
+            const bool nan = (ray.ox != ray.ox) || (ray.oy != ray.oy) || (ray.oz != ray.oz) || (ray.dx != ray.dx) ||
+                             (ray.dy != ray.dy) || (ray.dz != ray.dz);
             if (nan || p.node_count == 0) {
                 if (lane8 == 0) {
                     if (ANY)
                         p.occluded[rid] = 0;
                     else
-                        store_hit(p.hits, rid, bt, 0.f, 0.f, RTBVH_MISS);
+                        store_hit(p.hits, rid, ray.bt, 0.f, 0.f, RTBVH_MISS);
                 }
                 rid += stride;
                 continue;
             }
             active = true;
-            const uint32_t signs = (__float_as_uint(ix) >> 31) |
-                                   ((__float_as_uint(iy) >> 31) << 1) |
-                                   ((__float_as_uint(iz) >> 31) << 2);
-            const uint32_t flat = (fabsf(ix) > 3.4028235e38f ? 1u : 0u) |
-                                  (fabsf(iy) > 3.4028235e38f ? 2u : 0u) |
-                                  (fabsf(iz) > 3.4028235e38f ? 4u : 0u);
+            const uint32_t signs = (__float_as_uint(ray.ix) >> 31) |
+                                   ((__float_as_uint(ray.iy) >> 31) << 1) |
+                                   ((__float_as_uint(ray.iz) >> 31) << 2);
+            const uint32_t flat = (fabsf(ray.ix) > 3.4028235e38f ? 1u : 0u) |
+                                  (fabsf(ray.iy) > 3.4028235e38f ? 2u : 0u) |
+                                  (fabsf(ray.iz) > 3.4028235e38f ? 4u : 0u);
             oct = (signs & ~flat) | (flat << 3);
             ngx = BATCH ? scene_of_ray(p.ray_offsets, p.scene_count, uint32_t(rid)) : 0u;
             ngy = (1u << (24 + (oct & 7u))) | (1u << 16);
@@ -1015,11 +1219,11 @@ __global__ void __launch_bounds__(kGroupBlock) cw8_group_kernel(TraceParams p) {
         }
         bool overflow = false;
         bool found = false;
-        if (ngy >= kNodeGroup && group_bound(ngy) > bt) ngy = 0;
+        if (ngy >= kNodeGroup && group_bound(ngy) > ray.bt) ngy = 0;
         while (ngy < kNodeGroup && sp > 0) {
             --sp;
             const uint2 g = sp < kGroupLds ? lds[sp * (kGroupBlock / 8)] : deep[sp - kGroupLds];
-            if (group_bound(g.y) <= bt) {
+            if (group_bound(g.y) <= ray.bt) {
                 ngx = g.x;
                 ngy = g.y;
             }
@@ -1041,106 +1245,19 @@ __global__ void __launch_bounds__(kGroupBlock) cw8_group_kernel(TraceParams p) {
             }
             ngy = 0;
             if (idx < p.node_count) {
-                const uint4* q = reinterpret_cast<const uint4*>(p.cnodes + idx);
-                const uint8_t* planes = reinterpret_cast<const uint8_t*>(q + 2) + lane8;
-                // this lane's slot: near planes first along a positive direction
-                const uint32_t nx = (oct & 1u) ? 24u : 0u, ny = (oct & 2u) ? 32u : 8u,
-                               nz = (oct & 4u) ? 40u : 16u;
-                const uint32_t fx = 24u - nx, fy = 40u - ny, fz = 56u - nz;
-                const uint4 h0 = q[0], h1 = q[1];
-                const float qnx = float(planes[nx]), qfx = float(planes[fx]);
-                const float qny = float(planes[ny]), qfy = float(planes[fy]);
-                const float qnz = float(planes[nz]), qfz = float(planes[fz]);
-                const float stx = __uint_as_float((h0.w & 0xFFu) << 23);
-                const float sty = __uint_as_float(((h0.w >> 8) & 0xFFu) << 23);
-                const float stz = __uint_as_float(((h0.w >> 16) & 0xFFu) << 23);
-                float sx = stx * ix, sy = sty * iy, sz = stz * iz;
-                float bx = (__uint_as_float(h0.x) - ox) * ix;
-                float by = (__uint_as_float(h0.y) - oy) * iy;
-                float bz = (__uint_as_float(h0.z) - oz) * iz;
-                if (oct >= 8u) {
-                    if (oct & 8u) {
-                        sx = kFlatScale;
-                        bx = flat_offset((ox - __uint_as_float(h0.x)) / stx);
-                    }
-                    if (oct & 16u) {
-                        sy = kFlatScale;
-                        by = flat_offset((oy - __uint_as_float(h0.y)) / sty);
-                    }
-                    if (oct & 32u) {
-                        sz = kFlatScale;
-                        bz = flat_offset((oz - __uint_as_float(h0.z)) / stz);
-                    }
-                }
-                const float ex = fmaf(fabsf(sx), 255.0f, fabsf(bx)) * kBoxEps;
-                const float ey = fmaf(fabsf(sy), 255.0f, fabsf(by)) * kBoxEps;
-                const float ez = fmaf(fabsf(sz), 255.0f, fabsf(bz)) * kBoxEps;
-                const float tnx = fmaf(qnx, sx, bx - ex), tfx = fmaf(qfx, sx, bx + ex);
-                const float tny = fmaf(qny, sy, by - ey), tfy = fmaf(qfy, sy, by + ey);
-                const float tnz = fmaf(qnz, sz, bz - ez), tfz = fmaf(qfz, sz, bz + ez);
-                const float en = fmaxf(fmaxf(fmaxf(tnx, tny), tnz), tmin);
-                const bool hit = en <= fminf(fminf(fminf(tfx, tfy), tfz), bt);
-                const uint32_t hm = uint32_t(__ballot(hit) >> (threadIdx.x & 56u)) & 0xFFu;
-                const uint32_t imask = h0.w >> 24, lmask = h1.z & 0xFFu;
-                const uint32_t ih = hm & imask, th = hm & lmask;
-                const float gmin = min8(hit ? en : 3.0e38f);
-                if (ih) {
-                    ngx = h1.x;
-                    ngy = (oct_permute(ih, oct) << 24) | (imask << 16) | bound_bits(gmin);
-                }
-                if (th) {
-                    // every triangle hit at once, one per lane of its slot
-                    MtResult m;
-                    m.ok = false;
-                    uint32_t prim = RTBVH_MISS;
-                    if ((th >> lane8) & 1u) {
-                        const uint32_t pos =
-                            h1.y + uint32_t(__popc(lmask & ((1u << lane8) - 1u)));
-                        if (pos < p.index_count) {
-                            m = mt_prepared(p.tris, pos, ox, oy, oz, dx, dy, dz, tmin, &prim);
-                            m.ok = m.ok && prim != RTBVH_MISS &&
-                                   (ANY ? m.t < bt : lowest_first(m.t, prim, bt, bp));
-                        }
-                    }
-                    const uint32_t votes =
-                        uint32_t(__ballot(m.ok) >> (threadIdx.x & 56u)) & 0xFFu;
-                    if (votes) {
-                        if (ANY) {
-                            found = true;
-                            bp = 0;  // any id but RTBVH_MISS
-                        } else {
-                            // the lowest (t, id) of the group
-                            float t = m.ok ? m.t : __builtin_inff();
-                            uint32_t id = m.ok ? prim : RTBVH_MISS;
-                            uint32_t who = lane8;
-#pragma unroll
-                            for (int o = 1; o < 8; o <<= 1) {
-                                const float ot = __shfl_xor(t, o, 8);
-                                const uint32_t oid = __shfl_xor(id, o, 8);
-                                const uint32_t ow = __shfl_xor(who, o, 8);
-                                if (ot < t || (ot == t && oid < id)) {
-                                    t = ot;
-                                    id = oid;
-                                    who = ow;
-                                }
-                            }
-                            bt = t;
-                            bp = id;
-                            bu = __shfl(m.u, int(who), 8);
-                            bv = __shfl(m.v, int(who), 8);
-                        }
-                    }
-                }
+                uint32_t tgx = 0, tgy = 0;
+                group_node<ANY>(p, ray, idx, lane8, oct, ngx, ngy, tgx, tgy);
+                if (tgy) found = group_triangles<ANY>(p, ray, lane8, tgx, tgy);
             }
         }
         if (overflow && lane8 == 0) atomicOr(p.status, kStatusStackOverflow);
         if (found || overflow || (ngy < kNodeGroup && sp == 0)) {
             if (lane8 == 0) {
                 if (ANY)
-                    p.occluded[rid] = (bp != RTBVH_MISS) ? 1 : 0;
+                    p.occluded[rid] = (ray.bp != RTBVH_MISS) ? 1 : 0;
                 else
-                    store_hit(p.hits, rid, overflow ? __builtin_nanf("") : bt, bu, bv,
-                              overflow ? RTBVH_MISS : bp);
+                    store_hit(p.hits, rid, overflow ? __builtin_nanf("") : ray.bt, ray.bu, ray.bv,
+                              overflow ? RTBVH_MISS : ray.bp);
             }
             active = false;
             ngy = 0;

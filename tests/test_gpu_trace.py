@@ -345,3 +345,33 @@ def test_compressed_tree_over_ray_counts(rays_n):
     finally:
         rt.set_trace_config(None)
     tree.status()
+
+
+@pytest.mark.parametrize("rays_n", [98_305, 600_000, 1_200_000])
+def test_compressed_tree_long_rays_end_in_groups(rays_n):
+    """A wave's last eight rays are taken over by groups of eight lanes: rays
+    along a fan of slivers visit hundreds of nodes while the others miss, in
+    the one-ray-per-lane schedule and in runs, with stacks in LDS and (depth
+    0) in private memory."""
+    fan = scenes.noisy_sphere(400, 60, seed=41)  # slivers around both poles
+    verts = np.concatenate([fan, scenes.random_soup(200, 0.1, seed=42)]) * np.float32(8.0)
+    aabbs, centers = prep(verts)
+    dv = _dev(verts)
+    tree = rt.Builder(_dev(centers), aabbs=_dev(flat(aabbs))) \
+        .construct_locally_ordered_clustered().trace_tree(dv)
+    rays8 = ray_set(verts, rays_n, seed=43, kind="box")
+    rays8[:, 4:7] = (0.0, 0.0, 1.0)  # parallel to the axis through the poles
+    rays8[::997, 0:2] = np.float32(4.0)  # and some through them
+    check = np.unique(np.concatenate([np.arange(0, rays_n, 997), np.arange(0, rays_n, 61)]))
+    want = ref.trace_brute(verts, as_rays(rays8[check]), threads=8)
+    dr = _dev(rays8)
+    try:
+        for shape in (None, (64, 0, 800, 0, 16, 1), (128, 8, 1600, 0, 16, 0)):
+            rt.set_trace_config(None) if shape is None else rt.set_trace_config(*shape)
+            got = tree.intersect(dr).cpu().numpy().view(ref.HIT).reshape(-1)
+            assert hits_equal(got[check], want).all(), shape
+            occ = tree.occluded(dr).cpu().numpy()
+            assert np.array_equal(occ, (got["prim"] != 0xFFFFFFFF).astype(np.uint8)), shape
+    finally:
+        rt.set_trace_config(None)
+    tree.status()
