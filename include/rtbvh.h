@@ -33,9 +33,10 @@
  *
  * Memory: the builders behind create_bvh, rtbvh_gpu_create_bvh,
  * rtbvh_gpu_create_spatial_bvh, rtbvh_gpu_create_batch and
- * rtbvh_gpu_create_trace_tree*, and traversals with RTBVH_TRACE_ORDER_RAYS,
- * keep their scratch between calls, one block per kind (PLOC, binned SAH,
- * spatial SAH, traversal tree, ray order) and device, grown to the largest
+ * rtbvh_gpu_create_trace_tree*, traversals with RTBVH_TRACE_ORDER_RAYS, and
+ * rtbvh_gpu_adjoint* of 2^19 rays or more (outside stream capture) keep their
+ * scratch between calls, one block per kind (PLOC, binned SAH, spatial SAH,
+ * traversal tree, ray order, adjoint) and device, grown to the largest
  * request up to 1 GiB each and held until the process ends; concurrent
  * calls on one device and larger requests allocate and free their own.
  */
