@@ -129,9 +129,149 @@ __device__ __forceinline__ uint32_t scene_of_ray(const uint32_t* off, uint32_t s
     return lo;
 }
 
+// The other lanes' values of a group of four, in the order xor 1, 2, 3.
+template <int CTRL>
+__device__ __forceinline__ uint32_t quad_get(uint32_t x) {
+    return uint32_t(__builtin_amdgcn_update_dpp(0, int(x), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ uint32_t below_in_quad(uint32_t key) {
+    return (quad_get<0xB1>(key) < key ? 1u : 0u) + (quad_get<0x4E>(key) < key ? 1u : 0u) +
+           (quad_get<0x1B>(key) < key ? 1u : 0u);
+}
+
+// The rest of a ray of mbvh_fast_kernel by four lanes, a slot each (lane4):
+// the leaf slots are tested at once and accepted in the order of their
+// distances with the kernel's re-check, and the interior slots are pushed in
+// that order, so visits and result are the kernel's.  ls: the stack of the
+// ray's lane; deep: unused so far, filled alike by the four lanes.  Triangles
+// from the caller's vertex array.
+template <bool ANY>
+__device__ void mbvh_quad_rest(const TraceParams& p, const LdsStack& ls, DeepStack& deep, int sp,
+                               int32_t cur, uint32_t lane4, uint64_t rid, float ox, float oy,
+                               float oz, float dx, float dy, float dz, float ix, float iy,
+                               float iz, float tmin, float bt, float bu, float bv, uint32_t bp) {
+    float lox, loy, loz, hox, hoy, hoz;
+    slab_origin(ox, ix, lox, hox);
+    slab_origin(oy, iy, loy, hoy);
+    slab_origin(oz, iz, loz, hoz);
+    bool overflow = false;
+    for (;;) {
+        if (cur < 0) {
+            while (sp > 0) {
+                int32_t c;
+                float t;
+                stack_pop(ls, deep, sp, c, t);
+                if (t <= bt) {
+                    cur = c;
+                    break;
+                }
+            }
+        }
+        if (cur < 0 || uint32_t(cur) >= p.node_count) break;
+        const float* f = reinterpret_cast<const float*>(p.mnodes + cur) + lane4;
+        const float tx0 = (f[0] - lox) * ix, tx1 = (f[4] - hox) * ix;
+        const float ty0 = (f[8] - loy) * iy, ty1 = (f[12] - hoy) * iy;
+        const float tz0 = (f[16] - loz) * iz, tz1 = (f[20] - hoz) * iz;
+        const int32_t c = __float_as_int(f[24]), n = __float_as_int(f[28]);
+        const float a = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fminf(tz0, tz1));
+        const float b = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fmaxf(tz0, tz1));
+        const bool h = (b >= a) && (a <= bt) && (b >= tmin);
+        const uint32_t key =
+            h ? ((__float_as_uint(a > 0.0f ? a : 0.0f) & ~3u) | lane4) : 0xFFFFFFFFu;
+        // this lane's leaf: its lowest (t, id)
+        float lt = __builtin_inff(), lu = 0.f, lv = 0.f;
+        uint32_t lid = RTBVH_MISS;
+        if (h && n >= 0) {
+            for (int32_t j = 0; j < n; ++j) {
+                const uint32_t pos = uint32_t(c) + uint32_t(j);
+                if (pos >= p.index_count) break;
+                const uint32_t prim = p.indices[pos];
+                if (prim >= p.prim_count) continue;
+                const float* v = p.verts + size_t(prim) * 9;
+                const MtResult m = mt_candidate(v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7],
+                                                v[8], ox, oy, oz, dx, dy, dz, tmin);
+                if (!m.ok) continue;
+                if (ANY ? m.t < bt : lowest_first(m.t, prim, lt, lid)) {
+                    lt = m.t;
+                    lu = m.u;
+                    lv = m.v;
+                    lid = prim;
+                    if (ANY) break;
+                }
+            }
+        }
+        const uint32_t quad = threadIdx.x & 60u;  // first lane of the four
+        uint32_t found = uint32_t(__ballot(lid != RTBVH_MISS) >> quad) & 15u;
+        if (found) {
+            if (ANY) {
+                bp = 0;  // any id but RTBVH_MISS
+                break;
+            }
+            const uint32_t rank = below_in_quad(key);
+            for (uint32_t r = 0; r < 4; ++r) {
+                const uint32_t at =
+                    uint32_t(__ballot(lid != RTBVH_MISS && rank == r) >> quad) & 15u;
+                if (at == 0) continue;
+                const int who = int(__builtin_ctz(at));
+                const float t = __shfl(lt, who, 4), entry = __shfl(a, who, 4);
+                const uint32_t id = __shfl(lid, who, 4);
+                const float u = __shfl(lu, who, 4), v = __shfl(lv, who, 4);
+                if (entry <= bt && lowest_first(t, id, bt, bp)) {
+                    bt = t;
+                    bu = u;
+                    bv = v;
+                    bp = id;
+                }
+            }
+        }
+        // interior slots: the nearest is next, the others go far to near
+        const bool in = h && n < 0 && c >= 0 && a <= bt;
+        const uint32_t ins = uint32_t(__ballot(in) >> quad) & 15u;
+        cur = -1;
+        if (ins == 0) continue;
+        const int more = __popc(ins) - 1;
+        if (sp + more > RTBVH_MAX_STACK) {
+            overflow = true;
+            break;
+        }
+        // every lane of the four takes part: a lane exchange under a condition
+        // would read lanes that are switched off
+        const uint32_t before = below_in_quad(in ? key : 0xFFFFFFFFu);
+        const int place = in ? int(before) : 4;
+        const int first = __builtin_ctz(uint32_t(__ballot(place == 0) >> quad) & 15u);
+        if (sp + more <= ls.depth) {
+            if (in && place > 0) {
+                ls.i[(sp + more - place) * ls.stride] = c;
+                ls.t[(sp + more - place) * ls.stride] = a;
+            }
+            sp += more;
+            // the four lanes read each other's entries: keep the order
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            for (int k = more; k > 0; --k) {
+                const int who = __builtin_ctz(uint32_t(__ballot(place == k) >> quad) & 15u);
+                const int32_t ck = __shfl(c, who, 4);
+                const float ak = __shfl(a, who, 4);
+                (void)stack_push(ls, deep, sp, ck, ak);
+            }
+        }
+        cur = __shfl(c, first, 4);
+    }
+    if (lane4 != 0) return;
+    if (overflow) atomicOr(p.status, kStatusStackOverflow);
+    if (ANY)
+        p.occluded[rid] = (bp != RTBVH_MISS) ? 1 : 0;
+    else
+        store_hit(p.hits, rid, overflow ? __builtin_nanf("") : bt, bu, bv,
+                  overflow ? RTBVH_MISS : bp);
+}
+
 // BATCH: the MBVH is a forest whose node s is the root of scene s, and each
 // ray starts at the root of its scene.
-template <bool ANY, bool STATS, bool PREP, bool BATCH>
+// QUAD: a wave's last sixteen rays go to groups of four lanes
+// (mbvh_quad_rest), for launches of at most kQuadRays rays.
+template <bool ANY, bool STATS, bool PREP, bool BATCH, bool QUAD = false>
 __global__ void __launch_bounds__(kMaxBlock) mbvh_fast_kernel(TraceParams p) {
     if (p.gate && *p.gate) return;  // the tree this launch would read is incomplete
     extern __shared__ int32_t s_stack[];  // p.lds_depth entries per lane: ids, then distances
@@ -151,8 +291,38 @@ __global__ void __launch_bounds__(kMaxBlock) mbvh_fast_kernel(TraceParams p) {
     int32_t cur = -1;
     bool active = false;
     for (;;) {
+        const bool live = active || rid < p.ray_count;
+        const uint64_t lives = QUAD ? __ballot(live) : 0;
+        if (QUAD && lives == 0) break;
+        // the wave's last rays, all in hand
+        if (QUAD && __popcll(lives) <= 16 &&
+            __ballot(live && (!active || rid + stride < p.ray_count || sp > ls.depth)) == 0) {
+            const uint32_t lane = threadIdx.x & 63u;
+            uint64_t rest = lives;
+            for (uint32_t g = 0; g < lane >> 2; ++g) rest &= rest - 1;
+            const int own = rest ? __builtin_ctzll(rest) : 0;
+            const int32_t other = own - int(lane);
+            const LdsStack los{ls.i + other, ls.t + other, ls.depth, ls.stride};
+            const uint64_t at = (uint64_t(__shfl(uint32_t(rid >> 32), own, 64)) << 32) |
+                                __shfl(uint32_t(rid), own, 64);
+            const int osp = __shfl(sp, own, 64);
+            const int32_t ocur = __shfl(cur, own, 64);
+            const float v0 = __shfl(ox, own, 64), v1 = __shfl(oy, own, 64),
+                        v2 = __shfl(oz, own, 64), v3 = __shfl(dx, own, 64),
+                        v4 = __shfl(dy, own, 64), v5 = __shfl(dz, own, 64),
+                        v6 = __shfl(ix, own, 64), v7 = __shfl(iy, own, 64),
+                        v8 = __shfl(iz, own, 64), v9 = __shfl(tmin, own, 64),
+                        va = __shfl(bt, own, 64), vb = __shfl(bu, own, 64),
+                        vc = __shfl(bv, own, 64);
+            const uint32_t vd = __shfl(bp, own, 64);
+            if (rest != 0)  // whole groups
+                mbvh_quad_rest<ANY>(p, los, deep, osp, ocur, lane & 3u, at, v0, v1, v2, v3,
+                                          v4, v5, v6, v7, v8, v9, va, vb, vc, vd);
+            break;
+        }
+        if (QUAD && !live) continue;
         if (!active) {
-            if (rid >= p.ray_count) break;
+            if (!QUAD && rid >= p.ray_count) break;
             const float4* r4 = reinterpret_cast<const float4*>(p.rays + rid);
             const float4 ra = r4[0];
             const float4 rb = r4[1];
@@ -1285,12 +1455,19 @@ int current_dev() {
     return dev;
 }
 
+// Most rays of the 4-wide vertex path that use the QUAD kernel.  Its tail
+// takes 14 registers (5 waves per SIMD instead of 6): 2^18 camera rays on 20k
+// triangles 250 -> 152 us, 2^14 rays in the box 170 -> 115, 2^21 rays on 300k
+// triangles 2166 -> 1915 (box) and 599 -> 599 (camera), but 2^23 rays 6935 ->
+// 7380 and 1856 -> 2305.
+constexpr uint64_t kQuadRays = 3u << 19;
+
 template <bool ANY, bool STATS, bool PREP, bool BATCH = false, bool ITEM = false, bool CW8 = false,
-          bool IDS = false>
+          bool IDS = false, bool QUAD = false>
 hipError_t launch_fast(const TraceParams& p0, hipStream_t stream) {
     auto k = CW8 ? cw8_kernel<ANY, STATS, BATCH, IDS>
                  : (ITEM ? mbvh_item_kernel<ANY, STATS, BATCH>
-                         : mbvh_fast_kernel<ANY, STATS, PREP, BATCH>);
+                         : mbvh_fast_kernel<ANY, STATS, PREP, BATCH, QUAD>);
     const int dev = current_dev();
     const TraceConfig cfg = g_config_set[dev] ? g_config[dev] : default_trace_config();
     // resident blocks per CU for this shape, cached per (device, shape)
@@ -1409,6 +1586,10 @@ hipError_t launch_trace_fast(const TraceParams& p, bool any_hit, hipStream_t str
     if (p.tris)
         return any_hit ? launch_fast<true, false, true>(p, stream)
                        : launch_fast<false, false, true>(p, stream);
+    if (p.ray_count <= kQuadRays)
+        return any_hit ? launch_fast<true, false, false, false, false, false, false, true>(p, stream)
+                       : launch_fast<false, false, false, false, false, false, false, true>(p,
+                                                                                            stream);
     return any_hit ? launch_fast<true, false, false>(p, stream)
                    : launch_fast<false, false, false>(p, stream);
 }
