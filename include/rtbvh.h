@@ -376,8 +376,9 @@ typedef struct RTTraceConfig {
                                 that take new rays together, 1..64 */
     uint32_t schedule;       /* 4-wide kernel 0 and compressed trees: 0 each lane walks a
                                 fixed stride of rays, 1 the rays are dealt to the
-                                wavefronts in runs of 64 and a wavefront's lanes draw
-                                its next ray as they free up; the launcher lowers refill and the grid when
+                                wavefronts in runs of 64 (in one range each when the
+                                grid is 4 or more times the resident one) and a
+                                wavefront's lanes draw its next ray as they free up; the launcher lowers refill and the grid when
                                 the launch has few rays per resident lane, and runs
                                 schedule 0 with refill 1 below 2 rays per lane */
     uint32_t postpone;       /* compressed trees: a wavefront tests triangles only once this

@@ -41,7 +41,8 @@ struct TraceParams {
     uint32_t postpone;     // set by the launcher (compressed tree): triangle tests wait until
                            // this many lanes of the wave have one (0: never wait)
     bool small_leaves;     // every leaf holds at most 16 triangles (one-item kernel)
-    uint32_t wave_runs;    // set by the launcher: 1 rays dealt to the waves in runs (RaySchedule)
+    uint32_t wave_runs;    // set by the launcher: 1 rays dealt to the waves in runs, 2 in one
+                           // range each (RaySchedule)
     const uint32_t* ray_ids;  // non-null (compressed tree, one scene): position j traces ray
                               // ray_ids[j] and writes its result at ray_ids[j]
 };

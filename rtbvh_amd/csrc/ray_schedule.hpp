@@ -16,9 +16,15 @@ namespace rtbvh {
 // contiguous range per wave, the form before, left the waves of an image's
 // costly rows running alone at the end: on a 1M tree (default shape, 64 rays
 // a run against one range) 2^22 / 2^24 camera rays 1344 / 2704 us against
-// 1600 / 4171, 2^24 / 2^26 bounce rays 7.86 / 28.3 ms against 8.42 / 31.3,
-// 2^24 shadow rays in the order of their origins on 4M triangles 8.37 ms
+// 1600 / 4171, 2^24 bounce rays 7.86 ms against 8.42, 2^24 shadow rays in the order of their origins on 4M triangles 8.37 ms
 // against 11.39.  Runs of 128 to 512 rays: 1380 to 1558 us for the first.
+// A grid of many times the resident waves keeps one contiguous range per wave
+// (wave_runs 2): its waves are short enough to balance by themselves, and
+// waves spread over the whole set share less of the caches' traffic (2^26
+// bounce rays of an 8192 x 8192 image 24.6 ms against 26.2 in runs, a batch of
+// 256 scenes with 328M rays 97 against 137 ms; bounce rays of a 16:9 image
+// whose many misses start anew at random points go the other way, 31.3 against
+// 28.3 ms).
 constexpr uint32_t kRunShift = 6;
 
 // A value known to be equal in every lane of the wave, read from the first
@@ -45,10 +51,17 @@ struct RaySchedule {
         runs = p.wave_runs != 0;
         const uint64_t waves = (stride + 63) >> 6, wave = wave_uniform(tid >> 6);
         const uint64_t total = (p.ray_count + (1u << kRunShift) - 1) >> kRunShift;
-        base = wave << kRunShift;
-        jump = waves << kRunShift;
         cursor = 0;
-        end = wave < total ? uint32_t((total - wave + waves - 1) / waves) << kRunShift : 0u;
+        if (p.wave_runs == 2) {  // one range: its runs follow each other
+            const uint64_t per = (p.ray_count + waves - 1) / waves;
+            base = wave * per < p.ray_count ? wave * per : p.ray_count;
+            jump = uint64_t(1) << kRunShift;
+            end = uint32_t(p.ray_count - base < per ? p.ray_count - base : per);
+        } else {
+            base = wave << kRunShift;
+            jump = waves << kRunShift;
+            end = wave < total ? uint32_t((total - wave + waves - 1) / waves) << kRunShift : 0u;
+        }
         end = uint32_t(__builtin_amdgcn_readfirstlane(int(end)));
     }
 

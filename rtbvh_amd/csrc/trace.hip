@@ -460,6 +460,7 @@ int scheduled_grid(K kernel, TraceParams& p) {
     if (p.wave_runs) {
         blocks = need / (p.refill > 8 ? p.refill : 8u);
         blocks = blocks < resident ? resident : (blocks > 8 * resident ? 8 * resident : blocks);
+        if (blocks >= 4 * resident) p.wave_runs = 2u;
     }
     return int(need < blocks ? need : blocks);
 }

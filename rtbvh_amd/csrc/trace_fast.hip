@@ -1512,7 +1512,7 @@ hipError_t launch_fast(const TraceParams& p0, hipStream_t stream) {
     p.lds_depth = cfg.lds_depth;
     p.refill = refill;
     p.postpone = cfg.postpone;
-    p.wave_runs = runs ? 1u : 0u;
+    p.wave_runs = runs ? (blocks >= 4 * resident ? 2u : 1u) : 0u;
     hipLaunchKernelGGL(k, dim3(grid), dim3(cfg.block), lds, stream, p);
     return hipGetLastError();
 }

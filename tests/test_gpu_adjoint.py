@@ -231,7 +231,8 @@ def test_trace_tree_snapshot_guard():
 
 @pytest.mark.parametrize("rays_n, prims", [((1 << 19) - 1, 65), (1 << 19, 64), (1 << 19, 65),
                                            ((1 << 19) + 4097, 3), ((1 << 19) + 4097, 1000),
-                                           ((1 << 22) + 5, 70_001), (1 << 20, 1_048_577)])
+                                           ((1 << 22) + 5, 70_001), (1 << 20, 1_048_576),
+                                           (1 << 20, 1_048_577)])
 def test_vertex_gradients_of_many_rays(rays_n, prims):
     """From 2^19 rays on the vertex terms go through buckets of triangles (64
     to a bucket up to 65,536 triangles, then 128 and more; above 1,048,576 they
