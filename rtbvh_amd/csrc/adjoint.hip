@@ -209,10 +209,11 @@ __device__ __forceinline__ float sum8(float x) {
 // bucket, kSubChunk at a time: the records are placed in LDS in the order of
 // their triangles (a count, a scan, a scatter), a group of 8 lanes sums each
 // triangle's nine terms, and a bucket's sums, kept in LDS by their groups, are
-// added to the gradients at its end: plainly when the chunk holds the whole
-// bucket, by atomics otherwise.  Adding the terms by LDS atomics instead (nine
-// a record) took 195 us for 2^22 records, 51 us this
-// way.
+// added to the gradients at its end.  By atomics, also where the chunk holds
+// the whole bucket: calls on other streams may be adding to the same
+// gradients (rtbvh_gpu_adjoint accumulates), in either form.  Adding the terms
+// by LDS atomics instead (nine a record) took 195 us for 2^22 records, 51 us
+// this way.
 constexpr uint32_t kSubChunk = 2 * kSumBlock;
 
 __global__ void __launch_bounds__(kSumBlock)
@@ -241,7 +242,6 @@ __global__ void __launch_bounds__(kSumBlock)
     }
     uint32_t at = first;
     for (uint32_t b = lo; b < buckets && at < end; ++b) {
-        const uint32_t start = offsets[size_t(b) * tiles];
         const uint32_t next = b + 1 < buckets ? offsets[size_t(b + 1) * tiles] : count;
         const uint32_t stop = next < end ? next : end;
         if (stop <= at) continue;  // an empty bucket
@@ -306,14 +306,9 @@ __global__ void __launch_bounds__(kSumBlock)
         at = stop;
         float* g = a.grad_verts + size_t(b) * prims * 9;
         const uint32_t own = a.prim_count - b * prims < prims ? a.prim_count - b * prims : prims;
-        const bool whole = start >= first && next <= end;
         for (uint32_t k = threadIdx.x; k < own * 9; k += kSumBlock) {
             const float t = s_sum[k];
-            if (t == 0.f) continue;
-            if (whole)
-                g[k] += t;
-            else
-                atomicAdd(g + k, t);
+            if (t != 0.f) atomicAdd(g + k, t);
         }
         __syncthreads();
     }

@@ -25,6 +25,7 @@ from rtbvh_amd import scenes
 
 torch = pytest.importorskip("torch")
 import rtbvh_amd as rt  # noqa: E402
+from rtbvh_amd import _lib as L  # noqa: E402
 from rtbvh_amd import diff  # noqa: E402
 from rtbvh_amd.diff import trace_tuv  # noqa: E402
 
@@ -264,6 +265,67 @@ def test_vertex_gradients_of_many_rays(rays_n, prims):
     k.index_add_(0, idx, torch.ones(len(idx), dtype=torch.float64, device="cuda"))
     bound = (k[:, None] + 2.0) * 2.0 ** -24 * size
     assert bool(((d_v.double() - want).abs() <= bound).all())
+
+
+def _random_hits(verts, rays_n, seed):
+    """(rays, hits, gradients of t, u, v) of rays_n rays on random triangles
+    of verts.  A ray within 1e-5 of parallel to its triangle (the determinant
+    whose inverse scales lambda) is a miss, as the triangle test decides: one
+    of 786,432 rays on 40 triangles has 1.0e-7, which rounds to zero in 32
+    bits, so that no sum over it is finite."""
+    prims = verts.shape[0]
+    g = torch.Generator("cuda").manual_seed(seed)
+    rays = torch.rand((rays_n, 8), device="cuda", generator=g) + 0.1
+    hits = torch.rand((rays_n, 4), device="cuda", generator=g) * 0.5
+    prim = torch.randint(0, prims, (rays_n,), device="cuda", generator=g, dtype=torch.int32)
+    tri = verts.double().view(-1, 3, 3)[prim.long()]
+    normal = torch.linalg.cross(tri[:, 1] - tri[:, 0], tri[:, 2] - tri[:, 0])
+    prim[(normal * rays[:, 4:7].double()).sum(1).abs() < 1e-5] = -1
+    hits[:, 3] = prim.view(torch.float32)
+    return rays, hits, torch.randn((rays_n, 3), device="cuda", generator=g)
+
+
+def _add_adjoint(verts, rays, hits, grad, grad_verts, stream, origin=None):
+    """rtbvh_gpu_adjoint adding to grad_verts on `stream`."""
+    L.check(L.lib().rtbvh_gpu_adjoint(
+        verts.data_ptr(), verts.shape[0], rays.data_ptr(), hits.data_ptr(), rays.shape[0],
+        grad.data_ptr(), grad_verts.data_ptr(), origin.data_ptr() if origin is not None else None,
+        None, stream.cuda_stream), "rtbvh_gpu_adjoint")
+
+
+@pytest.mark.parametrize("prims", [40, 3000, 70_001])
+@pytest.mark.parametrize("counts", [(1 << 20,), (1 << 20, 1 << 18), (1 << 19, 3 << 18)])
+def test_calls_on_several_streams_add_to_one_gradient(counts, prims):
+    """The vertex gradients are added to what the buffer holds, also while
+    calls on other streams add to it: by buckets (2^19 rays or more) and by
+    single atomics at once.  The float32 sum of an initial value and k terms in
+    any order is within (k + 2) 2^-24 of the float64 sum, relative to the sum
+    of magnitudes."""
+    g = torch.Generator("cuda").manual_seed(prims)
+    verts = torch.rand((prims, 9), device="cuda", generator=g) * 4.0
+    start = torch.randn((prims, 9), device="cuda", generator=g)
+    got, want, size = start.clone(), start.double(), start.double().abs()
+    k = torch.zeros(prims, dtype=torch.float64, device="cuda")
+    calls = []
+    for c, rays_n in enumerate(counts):
+        rays, hits, grad = _random_hits(verts, rays_n, 100 * prims + c)
+        lam = torch.empty((rays_n, 3), device="cuda")
+        calls.append((rays, hits, grad, lam, torch.cuda.Stream()))
+    torch.cuda.synchronize()
+    for rays, hits, grad, lam, stream in calls:
+        _add_adjoint(verts, rays, hits, grad, got, stream, lam)
+    torch.cuda.synchronize()
+    for rays, hits, grad, lam, stream in calls:
+        prim = hits[:, 3].contiguous().view(torch.int32)
+        hit = prim >= 0
+        u, v, idx = hits[hit, 1], hits[hit, 2], prim[hit].long()
+        w = torch.stack([-((1.0 - u) - v), -u, -v], dim=1)
+        terms = (w[:, :, None] * lam[hit][:, None, :]).reshape(-1, 9).double()
+        want.index_add_(0, idx, terms)
+        size.index_add_(0, idx, terms.abs())
+        k.index_add_(0, idx, torch.ones(len(idx), dtype=torch.float64, device="cuda"))
+    bound = (k[:, None] + 2.0) * 2.0 ** -24 * size
+    assert bool(((got.double() - want).abs() <= bound).all())
 
 
 @pytest.mark.parametrize("n", [0, 1, 255, 257])
