@@ -5,6 +5,8 @@ the oracle and the reference's own FFI tests (rtbvh_ffi/src/lib.rs:851-1061).
 import ctypes
 import os
 import re
+import shutil
+import subprocess
 
 import numpy as np
 import pytest
@@ -45,6 +47,22 @@ def test_header_constants_match_the_binding():
     for name, value in pairs.items():
         assert defs.get(name) == value, name
     assert L.TRACE_ORDER_RAYS & L.TRACE_REFERENCE_ORDER == 0
+
+
+def test_every_persistent_kernel_has_its_own_resident_block_table():
+    """The grids of the binary and reference-order traversals come from the
+    blocks a device holds, looked up once per kernel and device: all kernels
+    have one function type, but not one occupancy, so each needs a table."""
+    if shutil.which("nm") is None:
+        pytest.skip("needs nm")
+    out = subprocess.run(["nm", L.lib()._name], check=True, capture_output=True, text=True).stdout
+    names = [line.split()[-1] for line in out.splitlines() if line]
+    kernels = {m.group(1) for n in names
+               for m in [re.search(r"__device_stub__(m?bvh_trace_kernelI\w+?EE)v", n)] if m}
+    tables = [n for n in names if "resident_blocks" in n and n.endswith("cached")]
+    assert len(kernels) >= 8
+    for kernel in kernels:  # a mangled name starts with its length
+        assert sum(re.search(r"\d" + kernel, t) is not None for t in tables) == 1, kernel
 
 
 def test_struct_layouts():
