@@ -363,8 +363,10 @@ void rtbvh_gpu_free_trace_tree(RTTraceTree tree);
 
 /* ---- Launch shape of the lowest-id MBVH traversal ---------------------------
  * (no counterpart in the reference).  Per device; the default is
- * {64, 8, 800, 0, 16, 1, 0}.  Results never depend on
- * it, only speed. */
+ * {64, 8, 800, 0, 16, 1, 0}.  Results never depend on it, only speed.
+ * Compressed trees trace up to 98,304 rays at a time with eight lanes a ray,
+ * in a shape of their own: there it applies to rays ordered by the library and
+ * to the _stats call, whose counts are those of one lane a ray, only. */
 typedef struct RTTraceConfig {
     uint32_t block;          /* threads per block: 64, 128 or 256 */
     uint32_t lds_stack;      /* traversal stack entries per ray kept in LDS, 0..32 */
@@ -398,7 +400,9 @@ ResultCode rtbvh_gpu_autotune_mbvh(RTMbvh mbvh, const RTRay *rays, size_t ray_co
                                    void *stream, RTTraceConfig *best);
 /* The same over a traversal tree; for a compressed (width 8) tree, 55 shapes:
  * schedule 1 with block 64/128 x LDS stack 6/8/10 x grid 400/800/1600 % x
- * refill 8/16/32, and the static schedule at 64/8/800 %. */
+ * refill 8/16/32, and the static schedule at 64/8/800 %.  Up to 98,304 rays
+ * against a compressed tree read no shape: they are traced once and the
+ * current shape stays (and is returned), so tune on a larger sample. */
 ResultCode rtbvh_gpu_autotune_trace_tree(RTTraceTree tree, const RTRay *rays, size_t ray_count,
                                          RTHit *hits, void *stream, RTTraceConfig *best);
 

@@ -321,6 +321,16 @@ ResultCode adjoint_entry(const float* vertices, size_t prim_count, const RTRay* 
     return Ok;
 }
 
+void store_config(const TraceConfig& c, RTTraceConfig* out) {
+    out->block = c.block;
+    out->lds_stack = c.lds_depth;
+    out->occupancy_pct = c.occupancy_pct;
+    out->kernel = c.kernel;
+    out->refill = c.refill;
+    out->schedule = c.schedule;
+    out->postpone = c.postpone;
+}
+
 // One pass over the rays (resp. hits) instead of a strided copy per field; at
 // 2^22 rays on the differentiable path 41 and 24 us, for about 340 us of copies, casts
 // and fills.
@@ -614,14 +624,7 @@ ResultCode rtbvh_gpu_get_trace_config(RTTraceConfig* config) {
         set_error("config must not be null");
         return Error;
     }
-    const TraceConfig c = get_trace_config();
-    config->block = c.block;
-    config->lds_stack = c.lds_depth;
-    config->occupancy_pct = c.occupancy_pct;
-    config->kernel = c.kernel;
-    config->refill = c.refill;
-    config->schedule = c.schedule;
-    config->postpone = c.postpone;
+    store_config(get_trace_config(), config);
     return Ok;
 }
 
@@ -632,7 +635,9 @@ namespace {
 
 // Times every candidate launch shape of `trace` (closest hit of the caller's
 // rays, best of two runs after a warm-up) and keeps the fastest as the
-// device's configuration.
+// device's configuration.  Rays that a compressed tree traces in groups of
+// lanes read no shape: they are traced once and the configuration stays, as
+// the candidates' times would differ by noise alone.
 template <typename Trace>
 ResultCode autotune(const RTRay* rays, size_t ray_count, RTHit* hits, void* stream,
                     RTTraceConfig* best, bool compressed, Trace trace) {
@@ -641,8 +646,16 @@ ResultCode autotune(const RTRay* rays, size_t ray_count, RTHit* hits, void* stre
         return Error;
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
+    hipError_t e = hipSuccess;
+    if (compressed && compressed_trace_by_groups(ray_count)) {
+        const ResultCode rc = trace();
+        if (rc != Ok) return rc;
+        if ((e = hipStreamSynchronize(st)) != hipSuccess) return hip_fail(e, "autotune");
+        if (best) store_config(get_trace_config(), best);
+        return Ok;
+    }
     hipEvent_t e0 = nullptr, e1 = nullptr;
-    hipError_t e = hipEventCreate(&e0);
+    e = hipEventCreate(&e0);
     if (e == hipSuccess) e = hipEventCreate(&e1);
     if (e != hipSuccess) {
         if (e0) (void)hipEventDestroy(e0);
@@ -701,15 +714,7 @@ ResultCode autotune(const RTRay* rays, size_t ray_count, RTHit* hits, void* stre
         return rc != Ok ? rc : hip_fail(e, "autotune");
     }
     set_trace_config(&top);
-    if (best) {
-        best->block = top.block;
-        best->lds_stack = top.lds_depth;
-        best->occupancy_pct = top.occupancy_pct;
-        best->kernel = top.kernel;
-        best->refill = top.refill;
-        best->schedule = top.schedule;
-        best->postpone = top.postpone;
-    }
+    if (best) store_config(top, best);
     return Ok;
 }
 

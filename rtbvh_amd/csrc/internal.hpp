@@ -66,6 +66,9 @@ TraceConfig default_trace_config();
 bool valid_trace_config(const TraceConfig& c);
 void set_trace_config(const TraceConfig* c);  // null: back to the default
 TraceConfig get_trace_config();
+// Closest and any hit of this many rays against a compressed tree run eight
+// lanes a ray, in a shape of their own.
+bool compressed_trace_by_groups(uint64_t ray_count);
 
 hipError_t launch_trace(const TraceParams& p, bool mbvh, bool ref_order, bool any_hit,
                         hipStream_t stream);

@@ -1538,13 +1538,15 @@ TraceConfig get_trace_config() {
     return g_config_set[dev] ? g_config[dev] : default_trace_config();
 }
 
+bool compressed_trace_by_groups(uint64_t ray_count) { return ray_count <= kGroupRays; }
+
 hipError_t launch_trace_fast(const TraceParams& p, bool any_hit, hipStream_t stream) {
     // rays read through an index: compressed trees, one scene, no counters
     if (p.ray_ids && (!p.cnodes || p.ray_offsets || p.stats)) return hipErrorInvalidValue;
     if (p.cnodes) {  // compressed 8-wide tree
         if (!p.tris || (p.stats && (any_hit || p.ray_offsets))) return hipErrorInvalidValue;
         // few rays: eight lanes each
-        if (p.ray_count <= kGroupRays && !p.stats && !p.ray_ids) {
+        if (compressed_trace_by_groups(p.ray_count) && !p.stats && !p.ray_ids) {
             if (p.ray_count == 0) return hipSuccess;
             if (p.ray_offsets)
                 return any_hit ? launch_group<true, true>(p, stream)

@@ -18,6 +18,7 @@ from tests.helpers import as_rays, flat, hits_equal, prep, ray_set, teapot
 
 torch = pytest.importorskip("torch")
 import rtbvh_amd as rt  # noqa: E402
+from rtbvh_amd import _lib as L  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -180,6 +181,45 @@ def test_batch_autotune_keeps_results():
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
         with pytest.raises(ValueError):
             rt.autotune(batch, rays)
+    finally:
+        rt.set_trace_config()
+
+
+@pytest.mark.parametrize("per_scene", [600, 20_000])
+def test_autotune_of_few_rays_keeps_the_shape(per_scene):
+    """A compressed tree traces up to 98,304 rays in a shape of their own: the
+    autotuner has nothing to time there and leaves the device's shape as it
+    is (postpone is 0 in every shape it tries), while it still writes the hits.
+    Above that it times the shapes, and every shape returns the same hits."""
+    vl = _scene_list()
+    batch, verts, offs = _build_batch(vl)
+    batch.attach_triangles(_dev(verts))
+    rays = _dev(np.concatenate([ray_set(v, per_scene, seed=60 + s, kind="box")
+                                for s, v in enumerate(vl)]))
+    roff = rt.SceneBatch.ray_offsets([per_scene] * len(vl), "cuda")
+    aabbs, centers = prep(vl[3])
+    dv = _dev(vl[3])
+    tree = rt.Builder(_dev(centers), aabbs=_dev(flat(aabbs))) \
+        .construct_locally_ordered_clustered().trace_tree(dv)
+    few = len(rays) <= 98_304
+    try:
+        for shape in ((128, 4, 400, 0, 8, 1, 16), (64, 10, 1600, 0, 32, 1, 3)):
+            rt.set_trace_config(*shape)
+            before = rt.get_trace_config()
+            want = batch.intersect(rays, roff)
+            for target, args in ((batch, (rays, roff)), (tree, (rays,))):
+                best = rt.autotune(target, *args)
+                assert best == rt.get_trace_config()
+                assert (best == before) == few, (shape, best)
+                assert torch.equal(batch.intersect(rays, roff).view(torch.int32),
+                                   want.view(torch.int32))
+                rt.set_trace_config(*shape)
+        hits = torch.zeros_like(want)
+        c = L.RTTraceConfig()
+        L.check(L.lib().rtbvh_gpu_autotune_batch(
+            batch._h, rays.data_ptr(), roff.data_ptr(), len(rays), hits.data_ptr(),
+            torch.cuda.current_stream().cuda_stream, c), "rtbvh_gpu_autotune_batch")
+        assert torch.equal(hits.view(torch.int32), want.view(torch.int32))
     finally:
         rt.set_trace_config()
 
