@@ -404,8 +404,9 @@ __global__ void __launch_bounds__(kBlock) bvh_trace_kernel(TraceParams p) {
         }
         if (left > 0) {
             found = test_leaf<REF, ANY>(p, item, 1, s);
-            // a leaf ends with the index array
-            left = uint32_t(++item) < p.index_count ? left - 1 : 0;
+            // a leaf ends with the index array: one that starts outside it
+            // (at -1, for instance) has no triangles
+            left = uint32_t(item++) < p.index_count ? left - 1 : 0;
         }
         if (left == 0) left = kNone;
         if (overflow) atomicOr(p.status, kStatusStackOverflow);

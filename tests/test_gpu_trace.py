@@ -314,6 +314,33 @@ def test_vertex_traversals_over_ray_counts_and_leaf_sizes(rays_n, per_leaf):
             assert np.array_equal(occ, (want["prim"] != 0xFFFFFFFF).astype(np.uint8)), mode
 
 
+@pytest.mark.parametrize("first, count, tested", [(-1, 3, 0), (-2, 4, 0), (1, 2, 2), (1, 7, 2),
+                                                  (3, 1, 0), (2, 1, 1)])
+def test_leaf_outside_the_index_array(first, count, tested):
+    """A leaf's triangles end with the index array, and a leaf that starts
+    outside it has none (src/iter.rs:337 skips missing primitives): at the
+    root and below it, in both tie rules and any hit."""
+    quad = np.array([[-1, -1, 1, 1, -1, 1, 0, 1, 1]], np.float32)
+    verts = np.repeat(quad, 3, axis=0)
+    idx = np.array([2, 1, 0], np.int32)
+    rays8 = np.array([[0, 0, 0, 1e-4, 0, 0, 1, 1e26]], np.float32)
+    box = np.zeros(3, ref.AABB)
+    box["min"], box["max"] = -2.0, 2.0
+    box["count"], box["left_first"] = [-1, 0, count], [1, 0, first]
+    leaf = box[2:].copy()
+    ids = idx[first:first + tested] if tested else []
+    for nodes in (leaf, box):
+        bvh = rt.Bvh.from_arrays(_dev(flat(nodes)), _dev(idx, torch.int32))
+        for ref_order in (False, True):
+            hit = _gpu_hits(bvh, verts, rays8, ref_order)["prim"][0]
+            if len(ids):
+                assert hit == (ids[0] if ref_order else min(ids))
+            else:
+                assert hit == 0xFFFFFFFF
+            occ = bvh.occluded(_dev(verts), _dev(rays8), reference_order=ref_order)
+            assert int(occ[0]) == (1 if len(ids) else 0)
+
+
 @pytest.mark.parametrize("rays_n", [1, 7, 9, 31, 33, 4097, 98_304, 98_305, 300_001])
 def test_compressed_tree_over_ray_counts(rays_n):
     """Up to 98,304 rays eight lanes hold a ray and test a node's triangles
