@@ -19,7 +19,7 @@ namespace rtbvh {
 // 1600 / 4171, 2^24 bounce rays 7.86 ms against 8.42, 2^24 shadow rays in the order of their origins on 4M triangles 8.37 ms
 // against 11.39.  Runs of 128 to 512 rays: 1380 to 1558 us for the first.
 // A grid of many times the resident waves keeps one contiguous range per wave
-// (wave_runs 2): its waves are short enough to balance by themselves, and
+// (wave_runs 2, the compressed and 4-wide traversals only): its waves are short enough to balance by themselves, and
 // waves spread over the whole set share less of the caches' traffic (2^26
 // bounce rays of an 8192 x 8192 image 24.6 ms against 26.2 in runs, a batch of
 // 256 scenes with 328M rays 97 against 137 ms; bounce rays of a 16:9 image

@@ -314,6 +314,55 @@ def test_vertex_traversals_over_ray_counts_and_leaf_sizes(rays_n, per_leaf):
             assert np.array_equal(occ, (want["prim"] != 0xFFFFFFFF).astype(np.uint8)), mode
 
 
+@pytest.mark.parametrize("any_hit", [False, True])
+def test_large_launches_equal_their_parts(any_hit):
+    """Rays are handed out by the size of the launch: a vertex traversal above
+    1,572,864 rays keeps one lane a ray to the end, the binary one deals runs
+    in up to 8 times the resident blocks (2^25 rays and more), and compressed
+    and 4-wide trees give each wave one range where the grid is 4 times the
+    resident one (from 2^24 rays, refilled by 8).  Every ray's result is that
+    of a launch of fewer rays."""
+    g = torch.Generator("cuda").manual_seed(5)
+    verts = _dev(np.concatenate([scenes.noisy_sphere(40, 30, seed=51),
+                                 scenes.random_soup(800, 0.1, seed=52)]))
+    aabbs, centers = prep(verts.cpu().numpy())
+    bvh = rt.Builder(_dev(centers), aabbs=_dev(flat(aabbs))).construct_locally_ordered_clustered()
+    mbvh = rt.Mbvh.from_bvh(bvh)
+    tree8, tree4 = bvh.trace_tree(verts), bvh.trace_tree(verts, width=4)
+    n = (1 << 25) + 321
+    rays = torch.rand((n, 8), device="cuda", generator=g)
+    rays[:, 3] = 1e-4
+    rays[:, 4:7] -= 0.5
+    rays[:, 7] = 1e30
+    rays[::3, 7] = 0.3
+
+    def check(name, fn, count, part):
+        whole = fn(rays[:count])
+        for b in range(0, count, part):
+            want = fn(rays[b:min(count, b + part)])
+            assert torch.equal(whole[b:b + part].view(torch.int32) if not any_hit
+                               else whole[b:b + part],
+                               want.view(torch.int32) if not any_hit else want), (name, b)
+        return whole
+
+    kind = "occluded" if any_hit else "intersect"
+    for ref_order in (False, True):
+        check("bvh", lambda r: getattr(bvh, kind)(verts, r, reference_order=ref_order), n, 5 << 20)
+    check("mbvh", lambda r: getattr(mbvh, kind)(verts, r), 1_600_003, 400_001)
+    check("mbvh", lambda r: getattr(mbvh, kind)(verts, r), 3 << 20, 3 << 19)
+    try:
+        rt.set_trace_config(64, 8, 3200, 0, 8, 1)
+        for tree in (tree8, tree4):
+            got = check(str(tree.width), getattr(tree, kind), n, 1 << 20)
+            if any_hit:
+                assert torch.equal(got, bvh.occluded(verts, rays))
+            else:
+                assert torch.equal(got.view(torch.int32), bvh.intersect(verts, rays)
+                                   .view(torch.int32))
+    finally:
+        rt.set_trace_config(None)
+
+
 @pytest.mark.parametrize("first, count, tested", [(-1, 3, 0), (-2, 4, 0), (1, 2, 2), (1, 7, 2),
                                                   (3, 1, 0), (2, 1, 1)])
 def test_leaf_outside_the_index_array(first, count, tested):
