@@ -395,7 +395,8 @@ __global__ void __launch_bounds__(kBlock) bvh_trace_kernel(TraceParams p) {
                     overflow = !push(right_first ? make_int2(l.extra1, l.extra2)
                                                  : make_int2(r.extra1, r.extra2));
                 }
-                if (hl || hr) {
+                // a ray whose stack is full ends here, untested
+                if ((hl || hr) && !overflow) {
                     const int32_t c = right_first ? r.extra1 : l.extra1;
                     left = c > -1 ? c : kNode;
                     item = right_first ? r.extra2 : l.extra2;

@@ -363,6 +363,65 @@ def test_large_launches_equal_their_parts(any_hit):
         rt.set_trace_config(None)
 
 
+def _chains(depth):
+    """(binary nodes, 4-wide nodes) of a chain of `depth` interior nodes that
+    one ray along +z walks to the end, with one entry left on the stack by
+    every level: the sibling, an interior node without children, lies behind."""
+    box = np.zeros(2 * depth + 1, ref.AABB)
+    box["min"], box["max"] = -2.0, 10.0
+    box["count"], box["left_first"] = -1, -1
+    box["left_first"][0] = 1
+    box["left_first"][1:-2:2] = np.arange(3, 2 * depth, 2)
+    box["max"][2::2] = 9.0
+    box["min"][2::2] = -1.0
+    box["count"][-2], box["left_first"][-2] = 1, 0
+    quad = np.zeros(depth + 1, ref.MBVH)
+    for ax in "xyz":
+        quad[f"min_{ax}"], quad[f"max_{ax}"] = 3.0e38, 3.0e38
+        quad[f"min_{ax}"][:-1, 0:2], quad[f"max_{ax}"][:-1, 0:2] = -2.0, 10.0
+    quad["min_z"][:-1, 1] = 0.5  # the sibling is entered later
+    quad["children"], quad["counts"] = -1, -1
+    quad["children"][:-1, 0] = np.arange(1, depth + 1)
+    quad["children"][:-1, 1] = depth
+    quad["children"][-2, 0], quad["counts"][-2, 0] = 0, 1
+    return box, quad
+
+
+@pytest.mark.parametrize("rays_n", [3, 64, 1000])
+@pytest.mark.parametrize("depth", [2, 100, 255, 256, 257, 258, 300])
+def test_stack_limit(depth, rays_n):
+    """RTBVH_MAX_STACK (256) entries: the binary traversal holds the child in
+    hand beside the siblings of 254 levels, the 4-wide one 256 siblings; a ray
+    that needs more ends with t = NaN, no hit, and a sticky StackOverflow."""
+    verts = np.array([[-1, -1, 1, 1, -1, 1, 0, 1, 1]], np.float32)
+    idx = _dev(np.zeros(1, np.int32), torch.int32)
+    rays = _dev(np.repeat(np.array([[0, 0, 0, 1e-4, 0, 0, 1, 1e26]], np.float32), rays_n, axis=0))
+    box, quad = _chains(depth)
+    bvh = rt.Bvh.from_arrays(_dev(flat(box)), idx)
+    mbvh = rt.Mbvh.from_arrays(_dev(flat(quad)), idx)
+    try:
+        for tree, orders, most in ((bvh, (False, True), 255), (mbvh, (False,), 257)):
+            for lds in (8, 0, 32):
+                rt.set_trace_config(64, lds, 100)
+                for ref_order in orders:
+                    hits = tree.intersect(_dev(verts), rays, reference_order=ref_order)
+                    prim = hits.view(torch.int32)[:, 3]
+                    if depth <= most:
+                        tree.status()
+                        assert bool((prim == 0).all()) and bool((hits[:, 0] == 1.0).all())
+                    else:
+                        with pytest.raises(rt.RTBvhError, match="StackOverflow"):
+                            tree.status()
+                        assert bool((prim == -1).all()) and bool(hits[:, 0].isnan().all())
+                    occ = tree.occluded(_dev(verts), rays, reference_order=ref_order)
+                    assert bool((occ == (1 if depth <= most else 0)).all())
+                    if depth > most:
+                        with pytest.raises(rt.RTBvhError, match="StackOverflow"):
+                            tree.status()
+    finally:
+        rt.set_trace_config(None)
+
+
 @pytest.mark.parametrize("first, count, tested", [(-1, 3, 0), (-2, 4, 0), (1, 2, 2), (1, 7, 2),
                                                   (3, 1, 0), (2, 1, 1)])
 def test_leaf_outside_the_index_array(first, count, tested):
