@@ -363,6 +363,34 @@ def test_large_launches_equal_their_parts(any_hit):
         rt.set_trace_config(None)
 
 
+@pytest.mark.parametrize("rays_n", [5, 5_000, 300_001])
+@pytest.mark.parametrize("per_leaf", [1, 24])
+def test_vertex_traversal_with_any_stack_in_lds(rays_n, per_leaf):
+    """The last sixteen rays of a wave go to groups of four lanes, whose stack
+    starts in the LDS of the ray's lane and goes on in private memory: with 0
+    to 32 entries in LDS the results are the oracle's."""
+    verts = np.concatenate([scenes.noisy_sphere(40, 30, seed=55),
+                            scenes.random_soup(900, 0.15, seed=56)])
+    aabbs, centers = prep(verts)
+    bvh = rt.Builder(_dev(centers), aabbs=_dev(flat(aabbs)),
+                     primitives_per_leaf=per_leaf).construct_binned_sah()
+    mbvh = rt.Mbvh.from_bvh(bvh)
+    quads = mbvh.quad_nodes().cpu().numpy().view(ref.MBVH).reshape(-1)
+    idx = bvh.indices().cpu().numpy().view(np.uint32)
+    rays8 = ray_set(verts, rays_n, seed=57, kind="box")
+    rays8[::3, 7] = np.float32(0.4)
+    rays8[::7, 4] = 0.0
+    want = ref.trace_mbvh(quads, idx, verts, as_rays(rays8), mode=ref.MODE_LOWEST_ID, threads=8)
+    flags = (want["prim"] != 0xFFFFFFFF).astype(np.uint8)
+    try:
+        for block, depth in ((64, 0), (128, 1), (256, 2), (64, 4), (64, 32)):
+            rt.set_trace_config(block, depth, 100)
+            assert hits_equal(_gpu_hits(mbvh, verts, rays8, False), want).all(), depth
+            assert np.array_equal(mbvh.occluded(_dev(verts), _dev(rays8)).cpu().numpy(), flags)
+    finally:
+        rt.set_trace_config(None)
+
+
 def _chains(depth):
     """(binary nodes, 4-wide nodes) of a chain of `depth` interior nodes that
     one ray along +z walks to the end, with one entry left on the stack by
