@@ -47,6 +47,8 @@ def _pack_rays(origins, directions, t_min, t_max):
             and origins.is_contiguous() and directions.is_contiguous())
     if not same or not all(isinstance(x, (int, float)) for x in (t_min, t_max)):
         return rays_tensor(origins, directions, t_min, t_max)
+    # the kernel reads memory: a lazily negated view is not what it holds
+    origins, directions = origins.resolve_neg(), directions.resolve_neg()
     r = torch.empty((origins.shape[0], RAY_FLOATS), dtype=torch.float32, device=origins.device)
     L.check(L.lib().rtbvh_gpu_pack_rays(_ptr(origins), _ptr(directions), r.shape[0], float(t_min),
                                         float(t_max), _ptr(r), _stream(r)), "rtbvh_gpu_pack_rays")
@@ -89,7 +91,9 @@ class TraceTUV(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gt, gu, gv, _gprim):
         verts, rays, hits = ctx.saved_tensors
-        parts = [None if g is None else g.contiguous() for g in (gt, gu, gv)]
+        # resolve_neg: complex losses hand back lazily negated views, whose
+        # memory holds the opposite sign
+        parts = [None if g is None else g.resolve_neg().contiguous() for g in (gt, gu, gv)]
         for name, x in (("vertices", verts), ("rays", rays), ("hits", hits),
                         *((f"grad_{k}", g) for k, g in zip("tuv", parts) if g is not None)):
             _require_device(x, name)

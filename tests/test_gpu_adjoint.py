@@ -355,6 +355,45 @@ def test_packed_rays_and_split_hits_equal_the_field_copies(n):
     assert prim.dtype == torch.int64 and torch.equal(prim, rt.hits_prim(hits))
 
 
+@pytest.mark.parametrize("n", [1, 2, 700])
+def test_lazily_negated_inputs_and_gradients(n):
+    """A complex loss gives a gradient that is a lazily negated view (for one
+    ray a contiguous one), and rays may be such views: values count, not what
+    the memory holds."""
+    verts = torch.tensor([[-4.0, -4.0, 0.0, 4.0, -4.0, 0.5, 0.0, 5.0, 1.0]], device="cuda")
+    aabbs, centers = scenes.triangle_aabbs_centers(verts.cpu().numpy())
+    bvh = rt.Builder(torch.from_numpy(centers).cuda(),
+                     aabbs=torch.from_numpy(aabbs).cuda()).construct_locally_ordered_clustered()
+    g = torch.Generator("cuda").manual_seed(n)
+    o = torch.rand((n, 3), device="cuda", generator=g) - torch.tensor([0.5, 0.5, 4.0]).cuda()
+    d = torch.rand((n, 3), device="cuda", generator=g) * 0.1 + torch.tensor([0, 0, 1.0]).cuda()
+    assert torch.equal(diff._pack_rays(torch._neg_view(o), torch._neg_view(d), 0.25, 7.5),
+                       rt.rays_tensor(-o, -d, 0.25, 7.5))
+    verts.requires_grad_(), o.requires_grad_(), d.requires_grad_()
+    t, u, v, prim = trace_tuv(bvh, verts, o, d)
+    assert bool((prim == 0).all())
+    weight = torch.complex(torch.rand(n, device="cuda", generator=g), torch.ones(n, device="cuda"))
+
+    def loss(a, b):
+        return (torch.complex(a, b).conj() * weight).abs().sum()
+
+    seen = []
+    u.register_hook(lambda x: seen.append(x.is_neg()))
+    got = torch.autograd.grad(loss(t, u), [verts, o, d])
+    assert seen == [True]
+    leaves = [x.detach().clone().requires_grad_() for x in (t, u)]
+    gt, gu = (x.resolve_neg() for x in torch.autograd.grad(loss(*leaves), leaves))
+    grad = torch.stack([gt, gu, torch.zeros_like(gt)], dim=1)
+    hits = torch.stack([t, u, v, prim.to(torch.int32).view(torch.float32)], 1).detach()
+    want = diff.adjoint(verts.detach(), rt.rays_tensor(o.detach(), d.detach()),
+                        hits.contiguous(), grad.contiguous())
+    assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
+    # the float atomics' order differs from run to run: (n + 2) 2^-24 of each
+    # magnitude, of which every term here is at most |dL/do|
+    size = want[1].abs().sum(0).repeat(3)
+    assert bool(((got[0] - want[0]).abs() <= 2 * (n + 2) * 2.0 ** -24 * size).all())
+
+
 def test_backward_of_one_output_and_of_expanded_gradients():
     """Gradients that autograd leaves out are zeros, and a sum's gradient is
     one number expanded over the rays (stride 0)."""
