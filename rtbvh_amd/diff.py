@@ -9,6 +9,7 @@ src/builders/spatial_sah.rs:132-163, is forward only).
 from __future__ import annotations
 
 import ctypes
+import math
 
 import torch
 
@@ -38,6 +39,15 @@ def adjoint(vertices: torch.Tensor, rays: torch.Tensor, hits: torch.Tensor,
     return gv, go, gd
 
 
+def _float32_number(x):
+    """A number that a 32-bit float takes as the general form stores it: not
+    beyond its range (refused there), nor an integer that is rounded twice."""
+    if isinstance(x, int):
+        return abs(x) <= 1 << 53
+    return isinstance(x, float) and (not math.isfinite(x)
+                                     or abs(x) <= torch.finfo(torch.float32).max)
+
+
 def _pack_rays(origins, directions, t_min, t_max):
     """rays_tensor in one pass where the library's kernel applies: contiguous
     (R, 3) float32 arrays on one device and plain numbers for t_min, t_max."""
@@ -45,7 +55,7 @@ def _pack_rays(origins, directions, t_min, t_max):
             and origins.dtype == directions.dtype == torch.float32
             and origins.device.type == "cuda" and origins.device == directions.device
             and origins.is_contiguous() and directions.is_contiguous())
-    if not same or not all(isinstance(x, (int, float)) for x in (t_min, t_max)):
+    if not same or not all(_float32_number(x) for x in (t_min, t_max)):
         return rays_tensor(origins, directions, t_min, t_max)
     # the kernel reads memory: a lazily negated view is not what it holds
     origins, directions = origins.resolve_neg(), directions.resolve_neg()

@@ -355,6 +355,25 @@ def test_packed_rays_and_split_hits_equal_the_field_copies(n):
     assert prim.dtype == torch.int64 and torch.equal(prim, rt.hits_prim(hits))
 
 
+@pytest.mark.parametrize("x", [1e39, -3.5e38, 1 << 70, 3.4028235e38, 3.4028234663852886e38,
+                               float("inf"), float("nan"), 1e-50, True, 7, (1 << 60) + (1 << 36) + 1,
+                               np.float64(0.1), np.float32(0.1)])
+def test_ray_ends_are_taken_or_refused_as_by_rays_tensor(x):
+    """t_min and t_max beyond the 32-bit range are refused, everything else is
+    rounded once, whichever form packs the rays."""
+    o, d = torch.rand((3, 3), device="cuda"), torch.rand((3, 3), device="cuda")
+
+    def packed(pack, *ends):
+        try:
+            return pack(o, d, *ends).view(torch.int32)
+        except Exception as e:
+            return type(e)
+
+    for ends in ((x, 7.5), (0.25, x)):
+        want, got = packed(rt.rays_tensor, *ends), packed(diff._pack_rays, *ends)
+        assert torch.equal(got, want) if isinstance(want, torch.Tensor) else got is want, ends
+
+
 @pytest.mark.parametrize("n", [1, 2, 700])
 def test_lazily_negated_inputs_and_gradients(n):
     """A complex loss gives a gradient that is a lazily negated view (for one
