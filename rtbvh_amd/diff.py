@@ -107,9 +107,14 @@ class TraceTUV(torch.autograd.Function):
         for name, x in (("vertices", verts), ("rays", rays), ("hits", hits),
                         *((f"grad_{k}", g) for k, g in zip("tuv", parts) if g is not None)):
             _require_device(x, name)
+        n, r = verts.reshape(-1, 9).shape[0], rays.shape[0]
+        # saved-tensor hooks may have handed back anything
+        if rays.shape != (r, RAY_FLOATS) or hits.shape != (r, 4) \
+                or any(g is not None and g.shape != (r,) for g in parts):
+            raise ValueError("the saved rays (R, 8) and hits (R, 4) and the gradients (R,) "
+                             "must agree")
         need_v = ctx.needs_input_grad[0]
         need_r = ctx.needs_input_grad[1] or ctx.needs_input_grad[2]
-        n, r = verts.numel() // 9, rays.shape[0]
         d_v = (torch.zeros((n, 9), dtype=torch.float32, device=verts.device) if need_v else None)
         d_o, d_d = ((torch.empty((r, 3), dtype=torch.float32, device=rays.device)
                      for _ in range(2)) if need_r else (None, None))

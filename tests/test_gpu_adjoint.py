@@ -374,6 +374,29 @@ def test_ray_ends_are_taken_or_refused_as_by_rays_tensor(x):
         assert torch.equal(got, want) if isinstance(want, torch.Tensor) else got is want, ends
 
 
+@pytest.mark.parametrize("cut", ["vertices", "rays", "hits"])
+def test_saved_tensors_of_another_shape_are_refused(cut):
+    """Saved-tensor hooks may hand back other tensors than were saved: shapes
+    that disagree are an error before anything is launched."""
+    verts = torch.rand((5, 9), device="cuda") * 4.0
+    aabbs, centers = scenes.triangle_aabbs_centers(verts.cpu().numpy())
+    bvh = rt.Builder(torch.from_numpy(centers).cuda(),
+                     aabbs=torch.from_numpy(aabbs).cuda()).construct_locally_ordered_clustered()
+    columns = {"vertices": 9, "rays": 8, "hits": 4}[cut]
+
+    def unpack(x):
+        if x.shape[-1] != columns:
+            return x
+        return x.reshape(-1)[:-1] if cut == "vertices" else x[:-1].contiguous()
+
+    verts.requires_grad_()
+    with torch.autograd.graph.saved_tensors_hooks(lambda x: x, unpack):
+        t, u, v, _ = trace_tuv(bvh, verts, torch.rand((7, 3), device="cuda"),
+                               torch.rand((7, 3), device="cuda"))
+    with pytest.raises((ValueError, RuntimeError)):
+        (t + u + v).sum().backward()
+
+
 @pytest.mark.parametrize("n", [1, 2, 700])
 def test_lazily_negated_inputs_and_gradients(n):
     """A complex loss gives a gradient that is a lazily negated view (for one
