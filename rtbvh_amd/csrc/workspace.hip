@@ -22,6 +22,15 @@ struct Slot {
 
 Slot g_slots[kMaxDevices][kWsKinds];
 
+// While it lives, this thread's allocations, frees and event calls leave alone
+// the captures that other threads have under way (in the default, global,
+// mode an allocation anywhere in the process invalidates them).
+struct BesideCaptures {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    BesideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~BesideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // The last stream-ordered user's work is complete (host wait).
 void settle(Slot& s) {
     if (s.pending) {
@@ -97,6 +106,7 @@ void workspace_release(Workspace* w, hipStream_t stream, bool wait) {
 // cannot serve is allocated here and freed by the release, which waits.
 hipError_t workspace_acquire_on(WorkspaceKind kind, size_t bytes, hipStream_t stream,
                                 Workspace* out) {
+    const BesideCaptures beside;
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) dev = -1;
     out->ptr = nullptr;
@@ -137,6 +147,7 @@ hipError_t workspace_acquire_on(WorkspaceKind kind, size_t bytes, hipStream_t st
 
 void workspace_release_on(Workspace* w, hipStream_t stream) {
     if (!w->ptr) return;
+    const BesideCaptures beside;
     if (w->cached) {
         Slot& s = g_slots[w->dev][w->kind];
         std::lock_guard<std::mutex> lk(s.mu);

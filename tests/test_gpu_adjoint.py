@@ -18,6 +18,8 @@ the gradient is pinned by mathematics, not by reference outputs:
     t is continuous there, u and v are not, so they are left out).
 Loss otherwise: L = sum over hit rays of w_t t + w_u u + w_v v, w ~ N(0, 1).
 """
+import threading
+
 import numpy as np
 import pytest
 
@@ -92,6 +94,57 @@ def _forward_backward(verts, rays, tree, w, dev):
     torch.cuda.synchronize()
     return (t.detach().cpu().numpy(), u.detach().cpu().numpy(), v.detach().cpu().numpy(),
             prim.cpu().numpy(), vt.grad.cpu().numpy(), o.grad.cpu().numpy(), d.grad.cpu().numpy())
+
+
+def test_calls_beside_a_capture_of_another_thread():
+    """A call of 2^19 rays or more takes a workspace: while another thread
+    records a graph (torch's default mode, in which an allocation anywhere
+    invalidates the recording) its first calls, which allocate and grow the
+    workspace, and later ones leave the recording alone.  The first test of
+    the file, so that nothing is allocated yet."""
+    print("[adjoint_beside_capture]", flush=True)
+    verts = torch.rand((100, 9), device="cuda") * 4.0
+    source = torch.rand(1000, device="cuda")
+    for rays_n in (1 << 19, 1 << 20, 1 << 20, 1 << 22):
+        rays, hits, grad = _random_hits(verts, rays_n, rays_n)
+        got, want = (torch.zeros((100, 9), device="cuda") for _ in range(2))
+        out = torch.zeros(1000, device="cuda")
+        torch.cuda.synchronize()
+        started, go, errors = threading.Event(), threading.Event(), []
+
+        def record():
+            try:
+                graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+                with torch.cuda.stream(stream):
+                    graph.capture_begin()
+                    try:
+                        torch.mul(source, 2.0, out=out)
+                        started.set()
+                        go.wait(60)
+                    finally:
+                        graph.capture_end()
+                for _ in range(3):
+                    out.zero_()
+                    torch.cuda.synchronize()
+                    graph.replay()
+                    torch.cuda.synchronize()
+                    assert torch.equal(out, source * 2.0)
+            except Exception as e:
+                errors.append(e)
+            finally:
+                started.set()
+
+        thread = threading.Thread(target=record)
+        thread.start()
+        started.wait(60)
+        try:
+            _add_adjoint(verts, rays, hits, grad, got, torch.cuda.current_stream())
+        finally:
+            go.set()
+            thread.join()
+        assert not errors, (rays_n, errors)
+        _add_adjoint(verts, rays, hits, grad, want, torch.cuda.current_stream())
+        assert torch.allclose(got, want, rtol=1e-4, atol=1e-4 * float(want.abs().max()))
 
 
 def test_adjoint_matches_fp64_gradient():
