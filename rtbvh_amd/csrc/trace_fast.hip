@@ -955,7 +955,8 @@ __device__ __forceinline__ bool group_triangles(const TraceParams& p, GroupRay& 
     return false;
 }
 
-template <bool ANY, bool STATS, bool BATCH, bool IDS = false>
+// TAIL: a wave's last eight rays go to groups of eight lanes.
+template <bool ANY, bool STATS, bool BATCH, bool IDS = false, bool TAIL = !STATS>
 __global__ void __launch_bounds__(kMaxBlock) __attribute__((amdgpu_waves_per_eu(8)))
 cw8_kernel(TraceParams p) {
     if (p.gate && *p.gate) return;  // the tree this launch would read is incomplete
@@ -999,7 +1000,7 @@ cw8_kernel(TraceParams p) {
         const uint64_t busy = __ballot(active);
         if (takers == 0 && busy == 0) break;  // wave-uniform: no ray left for any lane
         // the wave's last rays: a group of eight lanes takes each (below)
-        if (!STATS && takers == 0 && __popcll(busy) <= 8 && sched.last(p, active) &&
+        if (TAIL && takers == 0 && __popcll(busy) <= 8 && sched.last(p, active) &&
             __ballot(active && sp > ldepth) == 0) {
             group_busy = busy;
             break;
@@ -1213,7 +1214,7 @@ cw8_kernel(TraceParams p) {
             sched.next();
         }
     }
-    if (!STATS && group_busy != 0) {
+    if (TAIL && group_busy != 0) {
         // At most eight rays are left in the wave, and a ray that is long
         // after 64 others were not may visit thousands of nodes (a camera ray
         // along a sphere's pole).  2^20 / 2^22 camera rays on 1M triangles 1780 -> 690 /
@@ -1513,6 +1514,17 @@ hipError_t launch_fast(const TraceParams& p0, hipStream_t stream) {
     p.refill = refill;
     p.postpone = cfg.postpone;
     p.wave_runs = runs ? (blocks >= 4 * resident ? 2u : 1u) : 0u;
+    // Very large launches end in few long rays among many waves, and pay for
+    // the tail in every iteration instead: beside it the node step reads
+    // scalar registers back from vector lanes (10 a step for any hit by index,
+    // 2 without).  Without it ordered rays from 4 times the resident grid on
+    // (2^25 / 2^27 shadow rays on 1M triangles 21.2 -> 20.4 / 66.9 -> 62.8 ms,
+    // any hit 15.7 -> 15.3 / 54.2 -> 51.7), other closest hits from 8 times on
+    // (2^26 camera rays 17.11 -> 16.93 ms, of a 16:9 image 15.05 -> 14.85;
+    // at 2^25, 4 times, the tail is worth 6.51 -> 4.78).  Unordered any hit is
+    // the faster with it (2^26 bounce rays 24.8 against 25.1 ms).
+    if (CW8 && !STATS && (!ANY || IDS) && p.wave_runs == 2u && (IDS || blocks >= 8 * resident))
+        k = cw8_kernel<ANY, STATS, BATCH, IDS, false>;
     hipLaunchKernelGGL(k, dim3(grid), dim3(cfg.block), lds, stream, p);
     return hipGetLastError();
 }

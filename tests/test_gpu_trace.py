@@ -320,7 +320,8 @@ def test_large_launches_equal_their_parts(any_hit):
     1,572,864 rays keeps one lane a ray to the end, the binary one deals runs
     in up to 8 times the resident blocks (2^25 rays and more), and compressed
     and 4-wide trees give each wave one range where the grid is 4 times the
-    resident one (from 2^24 rays, refilled by 8).  Every ray's result is that
+    resident one (from 2^24 rays, refilled by 8), without a tail of groups for
+    ordered rays there and for closest hits at 8 times (2^25 rays).  Every ray's result is that
     of a launch of fewer rays."""
     g = torch.Generator("cuda").manual_seed(5)
     verts = _dev(np.concatenate([scenes.noisy_sphere(40, 30, seed=51),
@@ -354,6 +355,10 @@ def test_large_launches_equal_their_parts(any_hit):
         rt.set_trace_config(64, 8, 3200, 0, 8, 1)
         for tree in (tree8, tree4):
             got = check(str(tree.width), getattr(tree, kind), n, 1 << 20)
+            if tree is tree8:
+                ordered = getattr(tree, kind)(rays, order_rays=True)
+                assert torch.equal(ordered if any_hit else ordered.view(torch.int32),
+                                   got if any_hit else got.view(torch.int32))
             if any_hit:
                 assert torch.equal(got, bvh.occluded(verts, rays))
             else:
