@@ -380,8 +380,9 @@ typedef struct RTTraceConfig {
                                 fixed stride of rays, 1 the rays are dealt to the
                                 wavefronts in runs of 64 (in one range each when the
                                 grid is 4 or more times the resident one) and a
-                                wavefront's lanes draw its next ray as they free up; the launcher lowers refill and the grid when
-                                the launch has few rays per resident lane, and runs
+                                wavefront's lanes draw its next ray as they free up;
+                                the launcher lowers refill and the grid when the
+                                launch has few rays per resident lane, and runs
                                 schedule 0 with refill 1 below 2 rays per lane */
     uint32_t postpone;       /* compressed trees: a wavefront tests triangles only once this
                                 many of its lanes have one waiting, or a lane has nothing
@@ -413,7 +414,8 @@ ResultCode rtbvh_gpu_autotune_trace_tree(RTTraceTree tree, const RTRay *rays, si
  * o + t d = (1-u-v) v0 + u v1 + v v2.  Inputs (device): vertices (9 floats per
  * primitive), the rays and hits of the forward pass, grad_tuv (3 floats per
  * ray: dL/dt, dL/du, dL/dv).  Outputs (device, each may be NULL):
- * grad_vertices (9 floats per primitive) is ACCUMULATED into (zero it first),
+ * grad_vertices (9 floats per primitive) is ACCUMULATED into by atomics (zero
+ * it first; calls on several streams may add to one array at a time),
  * grad_origin / grad_direction (3 floats per ray) are written; rays that
  * missed get zeros. */
 ResultCode rtbvh_gpu_adjoint(const float *vertices, size_t prim_count, const RTRay *rays,

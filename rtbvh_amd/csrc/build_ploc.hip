@@ -63,19 +63,6 @@ struct Bounds6 {
     float mn[3], mx[3];
 };
 
-// v_min_f32 / v_max_f32 themselves: fminf and fmaxf put a canonicalising
-// v_max in front of every operand that comes from memory.
-__device__ __forceinline__ float vmin(float a, float b) {
-    float r;
-    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ float vmax(float a, float b) {
-    float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-
 // Nearest neighbour of cluster li of an LDS window of bounds (six arrays,
 // STRIDE apart, minima first): the lowest half_area(a.union_of(b))
 // (src/aabb.rs:74-86, 343-346) over the kRadius positions on either side, the

@@ -676,29 +676,6 @@ inline uint32_t sp_run(uint32_t tasks, uint32_t refs) {
     return std::max(64u, std::min(cap, refs / tasks));
 }
 
-// The instructions themselves: fminf / fmaxf put a canonicalising v_max in
-// front of every operand that comes from memory or a select.
-__device__ __forceinline__ float vmin(float a, float b) {
-    float r;
-    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ float vmax(float a, float b) {
-    float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ float vmin3(float a, float b, float c) {
-    float r;
-    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-__device__ __forceinline__ float vmax3(float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-
 // Where a triangle's edges cross one plane of axis u: whether any does, and
 // the bounds of the crossings on the other two axes (empty without one).
 struct Crossing {

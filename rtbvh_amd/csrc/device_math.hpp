@@ -23,6 +23,29 @@ __device__ __forceinline__ float ps_max(float a, float b) { return a > b ? a : b
 __device__ __forceinline__ float rs_min(float a, float b) { return (a != a) ? b : (b < a ? b : a); }
 __device__ __forceinline__ float rs_max(float a, float b) { return (a != a) ? b : (b > a ? b : a); }
 
+// v_min_f32 and its like themselves: fminf / fmaxf put a canonicalising v_max
+// in front of every operand that comes from memory or a select.
+__device__ __forceinline__ float vmin(float a, float b) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float vmax(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float vmin3(float a, float b, float c) {
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float vmax3(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
 struct alignas(16) DevAabb {
     float min[3];
     int32_t extra1;  // count

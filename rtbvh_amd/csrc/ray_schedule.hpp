@@ -16,15 +16,20 @@ namespace rtbvh {
 // contiguous range per wave, the form before, left the waves of an image's
 // costly rows running alone at the end: on a 1M tree (default shape, 64 rays
 // a run against one range) 2^22 / 2^24 camera rays 1344 / 2704 us against
-// 1600 / 4171, 2^24 bounce rays 7.86 ms against 8.42, 2^24 shadow rays in the order of their origins on 4M triangles 8.37 ms
-// against 11.39.  Runs of 128 to 512 rays: 1380 to 1558 us for the first.
+// 1600 / 4171, 2^24 bounce rays 7.86 ms against 8.42, 2^24 shadow rays in the
+// order of their origins on 4M triangles 8.37 ms against 11.39.  Runs of 128
+// to 512 rays: 1380 to 1558 us for the first.  Equal shares (the rays past
+// the last whole round of runs dealt in pieces of under 64) lost 1 % over 260
+// launches of 700k to 16M rays, 10 % on any hit of the binary traversal.
+//
 // A grid of many times the resident waves keeps one contiguous range per wave
-// (wave_runs 2, the compressed and 4-wide traversals only): its waves are short enough to balance by themselves, and
-// waves spread over the whole set share less of the caches' traffic (2^26
-// bounce rays of an 8192 x 8192 image 24.6 ms against 26.2 in runs, a batch of
-// 256 scenes with 328M rays 97 against 137 ms; bounce rays of a 16:9 image
-// whose many misses start anew at random points go the other way, 31.3 against
-// 28.3 ms).
+// (wave_runs 2, the compressed and 4-wide traversals only): waves spread over
+// the whole set share less of the caches' traffic (2^26 bounce rays of an
+// 8192 x 8192 image 24.6 ms against 26.2 in runs, a batch of 256 scenes with
+// 328M rays 97 against 137 ms).  Images whose costly part is small go the
+// other way: of a 16:9 image 2^26 camera rays 15.1 ms against 8.5 in runs and
+// its bounce rays, whose many misses start anew at random points, 31.3 against
+// 28.3.
 constexpr uint32_t kRunShift = 6;
 
 // A value known to be equal in every lane of the wave, read from the first

@@ -854,7 +854,6 @@ struct GroupRay {
 // Node idx against the ray, a slot per lane: its interior hits become the
 // node group in hand, its triangle hits (ngy and tgy stay 0 without any) the
 // triangle group.  The slot test is cw8_kernel's.
-template <bool ANY>
 __device__ __forceinline__ void group_node(const TraceParams& p, const GroupRay& r, uint32_t idx,
                                            uint32_t lane8, uint32_t oct, uint32_t& ngx,
                                            uint32_t& ngy, uint32_t& tgx, uint32_t& tgy) {
@@ -1289,7 +1288,7 @@ cw8_kernel(TraceParams p) {
                 }
                 ngy = 0;
                 if (idx < p.node_count)
-                    group_node<ANY>(p, r, idx, lane8, oct, ngx, ngy, tgx, tgy);
+                    group_node(p, r, idx, lane8, oct, ngx, ngy, tgx, tgy);
             }
             if (ngy < kNodeGroup && (tgy & 0xFFu) == 0u && sp == 0) break;
         }
@@ -1417,7 +1416,7 @@ __global__ void __launch_bounds__(kGroupBlock) cw8_group_kernel(TraceParams p) {
             ngy = 0;
             if (idx < p.node_count) {
                 uint32_t tgx = 0, tgy = 0;
-                group_node<ANY>(p, ray, idx, lane8, oct, ngx, ngy, tgx, tgy);
+                group_node(p, ray, idx, lane8, oct, ngx, ngy, tgx, tgy);
                 if (tgy) found = group_triangles<ANY>(p, ray, lane8, tgx, tgy);
             }
         }
@@ -1457,10 +1456,11 @@ int current_dev() {
 }
 
 // Most rays of the 4-wide vertex path that use the QUAD kernel.  Its tail
-// takes 14 registers (5 waves per SIMD instead of 6): 2^18 camera rays on 20k
-// triangles 250 -> 152 us, 2^14 rays in the box 170 -> 115, 2^21 rays on 300k
-// triangles 2166 -> 1915 (box) and 599 -> 599 (camera), but 2^23 rays 6935 ->
-// 7380 and 1856 -> 2305.
+// takes 14 registers (5 waves per SIMD instead of 6; any hit 12, 5 instead of
+// 7): 2^18 camera rays on 20k triangles 281 -> 193 us, 2^14 rays in the box
+// 170 -> 119, 1.57M rays on 300k triangles 1607 -> 1445 (box, any hit 1461 ->
+// 1335) and 654 -> 510 (camera, 542 -> 478), 2^21 rays 2166 -> 1915 (box) and
+// 599 -> 599 (camera), but 2^23 rays 6935 -> 7380 and 1856 -> 2305.
 constexpr uint64_t kQuadRays = 3u << 19;
 
 template <bool ANY, bool STATS, bool PREP, bool BATCH = false, bool ITEM = false, bool CW8 = false,

@@ -18,13 +18,9 @@
 // recorded into a graph.
 #include <vector>
 
-#include "block_scan.hpp"
 #include "internal.hpp"
 
 namespace rtbvh {
-
-hipError_t scan_exclusive_u32(uint32_t* data, uint32_t count, uint32_t* total, void* scratch,
-                              size_t scratch_bytes, hipStream_t stream);
 
 namespace {
 
