@@ -267,7 +267,7 @@ def run_adjoint(args, dev, rt, scenes, torch):
            "fp64_rel_error_200k_rays": {a: float(f"{b:.3e}") for a, b in errs.items()},
            "workload": "noisy sphere 250x200 quads (100k tris), 2^24 rays from radius 3 at the "
                        "cube [0.25, 0.75]^3, L = sum w t, w ~ N(0,1); forward = trace tree closest "
-                       "hit, backward = adjoint kernel (vertex grads by float atomics)"}
+                       "hit, backward = adjoint kernels (vertex grads summed through buckets of triangles)"}
     log(f"differentiable: forward {fm:.1f} ms, forward+backward {tm:.1f} ms, errors {errs}")
     del tree, bvh, verts, o, d, w
     torch.cuda.empty_cache()
