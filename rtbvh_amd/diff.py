@@ -39,13 +39,16 @@ def adjoint(vertices: torch.Tensor, rays: torch.Tensor, hits: torch.Tensor,
     return gv, go, gd
 
 
+_FLOAT32_MAX = torch.finfo(torch.float32).max
+
+
 def _float32_number(x):
     """A number that a 32-bit float takes as the general form stores it: not
     beyond its range (refused there), nor an integer that is rounded twice."""
     if isinstance(x, int):
         return abs(x) <= 1 << 53
     return isinstance(x, float) and (not math.isfinite(x)
-                                     or abs(x) <= torch.finfo(torch.float32).max)
+                                     or abs(x) <= _FLOAT32_MAX)
 
 
 def _pack_rays(origins, directions, t_min, t_max):
@@ -107,9 +110,9 @@ class TraceTUV(torch.autograd.Function):
         for name, x in (("vertices", verts), ("rays", rays), ("hits", hits),
                         *((f"grad_{k}", g) for k, g in zip("tuv", parts) if g is not None)):
             _require_device(x, name)
-        n, r = verts.reshape(-1, 9).shape[0], rays.shape[0]
+        (n, rest), r = divmod(verts.numel(), 9), rays.shape[0]
         # saved-tensor hooks may have handed back anything
-        if rays.shape != (r, RAY_FLOATS) or hits.shape != (r, 4) \
+        if rest or rays.shape != (r, RAY_FLOATS) or hits.shape != (r, 4) \
                 or any(g is not None and g.shape != (r,) for g in parts):
             raise ValueError("the saved rays (R, 8) and hits (R, 4) and the gradients (R,) "
                              "must agree")
